@@ -16,6 +16,7 @@
 // load of a wavefront one contiguous 256-byte (FP32) or 512-byte (FP64) segment.
 #pragma once
 
+#include "nc_iop.h"
 #include "nc_model.h"
 #include "nc_space.h"
 
@@ -138,22 +139,15 @@ struct RkErrEpilogue {
 };
 int64_t matvec_err_parts(const nc_matrix_s* A);  // row workgroups + sink rows
 void matvec_launch_err(nc_matrix_s* A, double t, const void* v, double* out, hipStream_t s, const RkErrEpilogue& epi);
-// Arnoldi projection sums computed by the mat-vec (nc_dual.h): besides out = A v, every
-// row workgroup writes the sums of its 512 rows, with v = V_{nv-1} and q = A v, into
-// part (value-major, nblk = the mat-vec's row workgroups). Time-invariant stored
-// generators with 2 rows per thread and 1..8 slots whose columns are all loaded or all
-// computed, unless plain mat-vecs are being timed; other generators take the separate
-// block pass.
-struct DualDots {
-  const void* V;     // V_0 .. V_{nv-1}, matrix precision, stride ld
-  int64_t ld;
-  int32_t nv;        // 1..32
-  const double* sc;  // scale of each V_i . q sum (null: 1)
-  double* part;
-  int64_t nblk;
-};
-bool matvec_dots_fusable(const nc_matrix_s* A);
-void matvec_launch_dots(nc_matrix_s* A, const void* v, double* out, hipStream_t s, const DualDots& d);
+// One column of the Krylov process (nc_iop.h) in one launch: V_c formed from q_{c-1} and the
+// two vectors before it while the mat-vec gathers it, q_c = A V_c and the column's sums.
+// Stored time-invariant generators at 2 rows per thread whose sink rows are not cut into
+// chunks, unless plain mat-vecs are being timed; other generators take the form / mat-vec /
+// sums kernels.
+bool matvec_krylov_fusable(const nc_matrix_s* A);
+void matvec_launch_krylov(nc_matrix_s* A, hipStream_t s, const IopArgs& p);
+// V_c over every row (the form kernel)
+void krylov_form(const IopArgs& p, bool fp32, hipStream_t s);
 // When kernel timing is on, hand out the next pair of HIP events for a dispatch-stamped
 // launch (the caller increments ev_used after the launch); false when timing is off.
 bool matvec_timing_slot(nc_matrix_s* A, hipEvent_t* e0, hipEvent_t* e1);

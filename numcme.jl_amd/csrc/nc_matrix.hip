@@ -18,7 +18,6 @@
 
 #include <mutex>
 
-#include "nc_dual.h"
 #include "nc_matrix.h"
 
 nc_matrix_s::~nc_matrix_s() {
@@ -418,12 +417,6 @@ struct MatArgs {
   double* err_part;
   double* err_ex;
   int32_t err_nex;
-  // Arnoldi projection sums (DOT kernels): basis V_0..V_{dot_nv-1} with stride dot_ld
-  const VT* dot_V;
-  int64_t dot_ld;
-  int32_t dot_nv;
-  const double* dot_sc;
-  double* dot_part;
 };
 
 template <typename T, int R>
@@ -826,12 +819,9 @@ __device__ __forceinline__ void stored_rows(const MatArgs<VT>& a, const VT* __re
 // Thread t owns state rows [R*t, R*t+R). Matrix streams are read with one R-wide vector
 // load per slot; v[i] and the predecessor gathers are scalar. EPI: the launch also forms
 // the next DP5(4) stage input (rk_epilogue) for its rows, state and sink rows alike.
-// DOT: the launch also writes the Arnoldi projection sums of its 512 rows (nc_dual.h):
-// the rows' q = A v and v go through LDS to the layout of the block sums, so the
-// projection pass need not read q back.
 // ERR: the launch also forms the DP5(4) error sums of its rows (err_row), one per row
 // workgroup and one per sink row, and the sink values of the event check.
-template <typename VT, typename OT, int KT, int R, int DM, bool EPI = false, bool DOT = false, bool ERR = false>
+template <typename VT, typename OT, int KT, int R, int DM, bool EPI = false, bool ERR = false>
 __global__ __launch_bounds__(kBlock) void k_matvec(MatArgs<VT> a, const VT* __restrict__ v, OT* __restrict__ out,
                                                    int accumulate) {
   const int64_t row_threads = (a.n + R - 1) / R;
@@ -843,32 +833,8 @@ __global__ __launch_bounds__(kBlock) void k_matvec(MatArgs<VT> a, const VT* __re
     const int64_t lb = x * q + (x < r8 ? x : r8) + (b >> 3);
     const int64_t t = lb * kBlock + threadIdx.x;
     const int64_t i0 = t * R;
-    if constexpr (DOT) {
-      static_assert(R * kBlock == kDualRows && DM <= 2 && !EPI, "projection epilogue: 2 rows per thread, stored generator");
-      __shared__ double s_x[kDualRows], s_y[kDualRows];
-      double vi[R] = {0.0, 0.0}, acc[R] = {0.0, 0.0};
-      if (i0 < a.n) stored_rows<VT, OT, KT, R, DM>(a, v, out, i0, accumulate, acc, vi);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const bool live = i0 + r < a.n;  // vi is already 0 past the states
-        s_x[R * threadIdx.x + r] = live ? acc[r] : 0.0;
-        s_y[R * threadIdx.x + r] = vi[r];
-      }
-      __syncthreads();
-      const int lane = threadIdx.x & 63;
-      double xx[8], yy[8];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          xx[4 * h + r] = s_x[256 * h + 4 * lane + r];
-          yy[4 * h + r] = s_y[256 * h + 4 * lane + r];
-        }
-      dual_block<VT>(a.dot_V, a.dot_ld, a.dot_nv, lb * kDualRows, xx, yy, a.dot_sc, a.dot_part, row_blocks, lb);
-      return;
-    }
     if constexpr (ERR) {
-      static_assert(DM <= 2 && !EPI && !DOT, "error epilogue: stored generator");
+      static_assert(DM <= 2 && !EPI, "error epilogue: stored generator");
       double r2 = 0.0;
       if (i0 < a.n) {
         double vi[R], acc[R];
@@ -922,7 +888,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec(MatArgs<VT> a, const VT* __re
       for (int u = 0; u < U; ++u) g[u] = (double)v[src[u]];
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (eb + (int64_t)u * kBlock < e1) acc += w[u] * g[u];
+        if (eb + (int64_t)u * kBlock < e1) acc = __fma_rn(w[u], g[u], acc);
     }
     __shared__ double part[kBlock / 64];
     __shared__ int s_last;
@@ -985,35 +951,18 @@ struct LaunchCfg {
   hipEvent_t e0, e1;
 };
 
-template <typename VT, typename OT, int K, int R, int DM, bool EPI = false, bool DOT = false, bool ERR = false>
+template <typename VT, typename OT, int K, int R, int DM, bool EPI = false, bool ERR = false>
 void launch_one(const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, OT* oo, int acc) {
   if (c.e0)
-    hipExtLaunchKernelGGL(k_matvec<VT, OT, K, R, DM, EPI, DOT, ERR>, dim3(c.grid), dim3(kBlock), 0, c.s, c.e0, c.e1, 0, a,
+    hipExtLaunchKernelGGL(k_matvec<VT, OT, K, R, DM, EPI, ERR>, dim3(c.grid), dim3(kBlock), 0, c.s, c.e0, c.e1, 0, a,
                           vv, oo, acc);
   else
-    k_matvec<VT, OT, K, R, DM, EPI, DOT, ERR><<<c.grid, kBlock, 0, c.s>>>(a, vv, oo, acc);
+    k_matvec<VT, OT, K, R, DM, EPI, ERR><<<c.grid, kBlock, 0, c.s>>>(a, vv, oo, acc);
 }
 
 // The error-epilogue kernels: FP64 output, 2 rows per thread, stored generator
 template <typename VT, int DM>
 void dispatch_err_kd(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, double* oo) {
-  switch (K) {
-    case 1: launch_one<VT, double, 1, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 2: launch_one<VT, double, 2, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 3: launch_one<VT, double, 3, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 4: launch_one<VT, double, 4, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 5: launch_one<VT, double, 5, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 6: launch_one<VT, double, 6, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 7: launch_one<VT, double, 7, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    case 8: launch_one<VT, double, 8, 2, DM, false, false, true>(c, a, vv, oo, 0); break;
-    default: launch_one<VT, double, 0, 2, 2, false, false, true>(c, a, vv, oo, 0); break;
-  }
-}
-
-// The projection-epilogue kernels: FP64 output, 2 rows per thread, every slot's column
-// loaded (DM 0) or every slot's computed (DM 1), at most 8 slots
-template <typename VT, int DM>
-void dispatch_dots_kd(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, double* oo) {
   switch (K) {
     case 1: launch_one<VT, double, 1, 2, DM, false, true>(c, a, vv, oo, 0); break;
     case 2: launch_one<VT, double, 2, 2, DM, false, true>(c, a, vv, oo, 0); break;
@@ -1022,7 +971,8 @@ void dispatch_dots_kd(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT*
     case 5: launch_one<VT, double, 5, 2, DM, false, true>(c, a, vv, oo, 0); break;
     case 6: launch_one<VT, double, 6, 2, DM, false, true>(c, a, vv, oo, 0); break;
     case 7: launch_one<VT, double, 7, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    default: launch_one<VT, double, 8, 2, DM, false, true>(c, a, vv, oo, 0); break;
+    case 8: launch_one<VT, double, 8, 2, DM, false, true>(c, a, vv, oo, 0); break;
+    default: launch_one<VT, double, 0, 2, 2, false, true>(c, a, vv, oo, 0); break;
   }
 }
 
@@ -1118,10 +1068,9 @@ void dispatch_r(int R, int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT
     dispatch_k<VT, OT, 1>(K, c, a, vv, oo, acc);
 }
 
+// The launch arguments every mat-vec form shares, at time t.
 template <typename VT>
-void launch_matvec_t(nc_matrix_s* A, double t, const void* v, void* out, bool accumulate, hipStream_t s,
-                     bool out_fp64, hipEvent_t e0, hipEvent_t e1, const RkEpilogue* epi = nullptr,
-                     const DualDots* dots = nullptr, const RkErrEpilogue* err = nullptr) {
+MatArgs<VT> mat_args(const nc_matrix_s* A, double t) {
   MatArgs<VT> a{};
   a.n = A->n;
   a.ld = A->ld;
@@ -1151,6 +1100,14 @@ void launch_matvec_t(nc_matrix_s* A, double t, const void* v, void* out, bool ac
   for (int r = 0; r < A->nr; ++r) a.sink_scale[r] = m->kinds[r] == NC_PROP_SEPARABLE ? m->tfactor(r, t) : 1.0;
   for (size_t q = 0; q < A->tv_r.size(); ++q)
     a.tv_scale[q] = A->tv_kind[q] == NC_PROP_SEPARABLE ? m->tfactor(A->tv_r[q], t) : 1.0;
+  return a;
+}
+
+template <typename VT>
+void launch_matvec_t(nc_matrix_s* A, double t, const void* v, void* out, bool accumulate, hipStream_t s,
+                     bool out_fp64, hipEvent_t e0, hipEvent_t e1, const RkEpilogue* epi = nullptr,
+                     const RkErrEpilogue* err = nullptr) {
+  MatArgs<VT> a = mat_args<VT>(A, t);
   // the matrix-free kernel takes 1 or 2 rows per thread (4 runs as 2)
   const int R = (out_fp64 && A->mf_mode && A->rows_per_thread == 4) ? 2 : A->rows_per_thread;
   const int64_t row_threads = (A->n + R - 1) / R;
@@ -1193,23 +1150,7 @@ void launch_matvec_t(nc_matrix_s* A, double t, const void* v, void* out, bool ac
     else if ((a.dia_mask & all) == all)
       dispatch_err_kd<VT, 1>(A->K, c, a, vv, reinterpret_cast<double*>(out));
     else
-      launch_one<VT, double, 0, 2, 2, false, false, true>(c, a, vv, reinterpret_cast<double*>(out), 0);
-    return;
-  }
-  if (dots) {
-    if (!matvec_dots_fusable(A) || accumulate || !out_fp64 || R != 2)
-      throw Error(NC_ERR_INTERNAL, "mat-vec projection epilogue not available");
-    if (dots->nv < 1 || dots->nv > 32 || dots->nblk != row_blocks)
-      throw Error(NC_ERR_INTERNAL, "projection blocks do not match the mat-vec's row workgroups");
-    a.dot_V = reinterpret_cast<const VT*>(dots->V);
-    a.dot_ld = dots->ld;
-    a.dot_nv = dots->nv;
-    a.dot_sc = dots->sc;
-    a.dot_part = dots->part;
-    if (a.dia_mask == 0u)
-      dispatch_dots_kd<VT, 0>(A->K, c, a, vv, reinterpret_cast<double*>(out));
-    else
-      dispatch_dots_kd<VT, 1>(A->K, c, a, vv, reinterpret_cast<double*>(out));
+      launch_one<VT, double, 0, 2, 2, false, true>(c, a, vv, reinterpret_cast<double*>(out), 0);
     return;
   }
   if (out_fp64 && A->mf_mode)
@@ -1218,6 +1159,284 @@ void launch_matvec_t(nc_matrix_s* A, double t, const void* v, void* out, bool ac
     dispatch_r<VT, double>(R, A->K, c, a, vv, reinterpret_cast<double*>(out), acc);
   else
     dispatch_r<VT, VT>(R, A->K, c, a, vv, reinterpret_cast<VT*>(out), acc);
+}
+
+// ---- Krylov column (nc_iop.h) ------------------------------------------------------------
+// V_c over every row from q_{c-1} and the two vectors before it
+template <typename BT>
+__global__ __launch_bounds__(kIopThreads) void k_krylov_form(IopArgs p) {
+  constexpr int R = 4;
+  const int c = p.c;
+  BT* V = reinterpret_cast<BT*>(p.V);
+  const BT* __restrict__ v1 = V + (int64_t)(c - 1) * p.ld;
+  const BT* __restrict__ v0 = V + (int64_t)(c > 1 ? c - 2 : 0) * p.ld;  // column 1: weight zero
+  const double* __restrict__ q = p.q[(c - 1) & 1];
+  BT* __restrict__ vn = V + (int64_t)c * p.ld;
+  const int64_t stride = (int64_t)gridDim.x * kIopThreads * R;
+  int64_t i = ((int64_t)blockIdx.x * kIopThreads + threadIdx.x) * R;
+  // the first rows' loads are in flight while the fold runs
+  int64_t ic = i < p.ld ? i : 0;
+  Pack<double, R> qv = ldpack<double, R>(q + ic);
+  Pack<BT, R> a = ldpack<BT, R>(v1 + ic), b = ldpack<BT, R>(v0 + ic);
+  __builtin_amdgcn_sched_barrier(0);
+  const IopCoef o = iop_finish_column<BT>(p, c - 1);
+  for (; i < p.ld; i += stride) {
+    if (i != ic) {
+      qv = ldpack<double, R>(q + i);
+      a = ldpack<BT, R>(v1 + i);
+      b = ldpack<BT, R>(v0 + i);
+    }
+    Pack<BT, R> w;
+#pragma unroll
+    for (int r = 0; r < R; ++r) w.v[r] = iop_row<BT>(o.xs, o.c1, o.c0, qv.v[r], a.v[r], b.v[r]);
+    *reinterpret_cast<Pack<BT, R>*>(vn + i) = w;
+  }
+}
+
+template <typename BT>
+void launch_form(const IopArgs& p, hipStream_t s) {
+  k_krylov_form<BT><<<std::min<unsigned>(kIopGroups, grid_for(p.ld / 4, kIopThreads)), kIopThreads, 0, s>>>(p);
+  NC_CHECK_HIP(hipGetLastError());
+}
+
+// What one thread loads for its two rows of a block: the matrix entries and, for the rows
+// and every predecessor, q_{c-1}, V_{c-1} and V_{c-2} (column 0: V_0 itself, in o1 / g1).
+template <typename VT, int KT>
+struct ColLoads {
+  Pack<double, 2> dg, oq;
+  Pack<VT, 2> o1, o0, w[KT];
+  Pack<double, 2> gq[KT];
+  Pack<VT, 2> g1[KT], g0[KT];
+};
+
+// Two consecutive elements at any element alignment, as one load
+template <typename T>
+__device__ inline Pack<T, 2> ldpair(const T* p) {
+  typedef T pair_t __attribute__((ext_vector_type(2), aligned(alignof(T))));
+  const pair_t v = *reinterpret_cast<const pair_t*>(p);
+  Pack<T, 2> o;
+  o.v[0] = v.x;
+  o.v[1] = v.y;
+  return o;
+}
+
+// Two consecutive elements past the caches' write allocation: the next launch reads them on
+// other XCDs, and what is still dirty in an L2 is written back at the kernel's end (plain
+// stores: 18.1 us a column on 1024^2 FP32 states, these 16.7).
+template <typename T>
+__device__ inline void stpair(T* p, T a, T b) {
+  typedef T pair_t __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store((pair_t){a, b}, reinterpret_cast<pair_t*>(p));
+}
+
+// A column's sink row r by one workgroup, its entries in k_matvec's order
+template <typename VT, bool STORED>
+__device__ inline void krylov_sink(const MatArgs<VT>& a, const IopArgs& p, int r, const VT* __restrict__ v1,
+                                   const VT* __restrict__ v0, VT* __restrict__ vn, const double* __restrict__ qp,
+                                   double* __restrict__ qn) {
+  double xs = 0.0, c1 = 1.0, c0 = 0.0;
+  if constexpr (!STORED) {
+    const IopCoef o = iop_finish_column<VT>(p, p.c - 1);
+    xs = o.xs, c1 = o.c1, c0 = o.c0;
+  }
+  auto form = [&](int64_t j) -> double {
+    return STORED ? (double)v1[j] : (double)iop_row<VT>(xs, c1, c0, qp[j], v1[j], v0[j]);
+  };
+  const int64_t n = a.n, e0 = a.sink_off[r], e1 = a.sink_off[r + 1];
+  double acc = 0.0;
+  if (threadIdx.x < kBlock)
+    for (int64_t e = e0 + threadIdx.x; e < e1; e += kBlock)
+      acc = __fma_rn((double)a.sink_val[e], form(a.sink_src[e]), acc);
+  __shared__ double part[kBlock / 64];
+  acc = wave_sum(acc);
+  if (threadIdx.x < kBlock && (threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int w = 0; w < kBlock / 64; ++w) s += part[w];
+    s *= a.sink_scale[r];
+    qn[n + r] = s;
+    if constexpr (!STORED) vn[n + r] = (VT)form(n + r);
+  }
+}
+
+// Column c of the Krylov process: V_c = xs q_{c-1} + c1 V_{c-1} + c0 V_{c-2} is formed where
+// it is gathered, so that the update pass, its launch and its re-read go: q_c = A V_c, V_c
+// stored for the workgroup's own rows, and the column's five sums. The coefficients come
+// from the previous column's partials, folded by every workgroup while its first loads are
+// in flight (2.7 us of a 512-group column, 0.3 us at 152 groups). 16.7 us on 1024^2 FP32
+// states for 54.6 MB (3.3 TB/s; Infinity Cache and the fold), 5.3 us on 301 x 259 FP64; the
+// mat-vec with projection, fold and update passes it replaces took 38 and 16 us. Forming V_c
+// by a pass of its own first (17.3 us), forming it once into an LDS tile with a halo (16.0;
+// 6 instead of 5.3 us on 301 x 259), two blocks' loads in flight (20.5) and 512 threads (24)
+// were measured.
+template <typename VT, int KT, int DM, bool STORED>
+__global__ __launch_bounds__(kIopThreads) void k_krylov_col(MatArgs<VT> a, IopArgs p) {
+  constexpr int KA = KT > 0 ? KT : 1;
+  const int c = p.c;
+  VT* V = reinterpret_cast<VT*>(p.V);
+  VT* __restrict__ vn = V + (int64_t)c * p.ld;
+  // formed: the two vectors V_c is formed from (column 1: v0 with weight zero); stored: V_c
+  // and the vector before it (column 0: not used)
+  const VT* __restrict__ v1 = V + (int64_t)(STORED ? c : c - 1) * p.ld;
+  const VT* __restrict__ v0 = V + (int64_t)(STORED ? max(c - 1, 0) : max(c - 2, 0)) * p.ld;
+  const double* __restrict__ qp = p.q[(c + 1) & 1];
+  double* __restrict__ qn = p.q[c & 1];
+  const int64_t n = a.n;
+  if ((int)blockIdx.x < p.groups) {
+    // one contiguous range of blocks per XCD, as in k_matvec
+    const int b = blockIdx.x, qd = p.groups >> 3, r8 = p.groups & 7, x8 = b & 7;
+    const int g = x8 * qd + (x8 < r8 ? x8 : r8) + (b >> 3);
+    const int64_t blk0 = (int64_t)g * p.nblk / p.groups, blk1 = (int64_t)(g + 1) * p.nblk / p.groups;
+    auto col_of = [&](int k, int64_t i0, int r, const Pack<int32_t, 2>& cl) -> int64_t {
+      const bool dia = DM == 1 || (DM == 2 && ((a.dia_mask >> k) & 1u));
+      if (!dia) return cl.v[r];
+      const int64_t j = i0 + r + a.dia_off[k];
+      return j < 0 ? 0 : (j > n - 1 ? n - 1 : j);
+    };
+    auto load = [&](int64_t blk, ColLoads<VT, KA>& l) {
+      int64_t i0 = blk * kIopRows + 2 * threadIdx.x;
+      i0 = i0 < n ? i0 : 0;  // past the states: a valid row, not used
+      l.dg = ldpack<double, 2>(a.diag + i0);
+      l.o1 = ldpack<VT, 2>(v1 + i0);
+      l.o0 = ldpack<VT, 2>(v0 + i0);
+      if constexpr (!STORED) l.oq = ldpack<double, 2>(qp + i0);
+      if constexpr (KT > 0) {
+#pragma unroll
+        for (int k = 0; k < KT; ++k) l.w[k] = ldpack<VT, 2>(a.val + k * a.ld + i0);
+        if constexpr (DM == 1) {
+          // Computed columns: the two rows' predecessors are neighbours, one load for both
+          // (scalar gathers of three vectors made the column 19.2 us on 1024^2 FP32
+          // states, pairs 18.1). Where the first row's would be -1 the pair is moved up by one;
+          // past the states it reads sink or padding rows, whose weight is zero.
+#pragma unroll
+          for (int k = 0; k < KT; ++k) {
+            const int64_t raw = i0 + a.dia_off[k], hi = p.ld - 2;  // rows past the states: padding
+            const int64_t j = raw < 0 ? 0 : (raw > hi ? hi : raw);
+            l.g1[k] = ldpair(v1 + j);
+            if constexpr (!STORED) {
+              l.gq[k] = ldpair(qp + j);
+              l.g0[k] = ldpair(v0 + j);
+            }
+          }
+        } else {
+          Pack<int32_t, 2> cl[KT];
+#pragma unroll
+          for (int k = 0; k < KT; ++k) cl[k] = ldpack<int32_t, 2>(a.col + k * a.ld + i0);
+#pragma unroll
+          for (int k = 0; k < KT; ++k)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+              l.g1[k].v[r] = v1[cl[k].v[r]];
+              if constexpr (!STORED) {
+                l.gq[k].v[r] = qp[cl[k].v[r]];
+                l.g0[k].v[r] = v0[cl[k].v[r]];
+              }
+            }
+        }
+      }
+    };
+    ColLoads<VT, KA> l;
+    load(blk0, l);
+    __builtin_amdgcn_sched_barrier(0);
+    double xs = 0.0, c1 = 1.0, c0 = 0.0;
+    if constexpr (!STORED) {
+      const IopCoef o = iop_finish_column<VT>(p, c - 1);
+      xs = o.xs, c1 = o.c1, c0 = o.c0;
+    }
+    double t[kIopSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int64_t blk = blk0; blk < blk1; ++blk) {
+      if (blk > blk0) {
+        load(blk, l);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const int64_t i0 = blk * kIopRows + 2 * threadIdx.x;
+      if (i0 >= n) continue;
+      double x[2], acc[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        x[r] = STORED ? (double)l.o1.v[r] : (double)iop_row<VT>(xs, c1, c0, l.oq.v[r], l.o1.v[r], l.o0.v[r]);
+        acc[r] = __dmul_rn(l.dg.v[r], x[r]);
+      }
+      if constexpr (KT > 0) {
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+          double gv[2];
+#pragma unroll
+          for (int r = 0; r < 2; ++r)
+            gv[r] = STORED ? (double)l.g1[k].v[r]
+                          : (double)iop_row<VT>(xs, c1, c0, l.gq[k].v[r], l.g1[k].v[r], l.g0[k].v[r]);
+          if (DM == 1 && i0 + a.dia_off[k] == -1) gv[1] = gv[0];  // the pair moved up by one
+#pragma unroll
+          for (int r = 0; r < 2; ++r) acc[r] = __fma_rn((double)l.w[k].v[r], gv[r], acc[r]);
+        }
+      } else {
+        for (int k = 0; k < a.K; ++k) {
+          const Pack<VT, 2> w = ldpack<VT, 2>(a.val + k * a.ld + i0);
+          const Pack<int32_t, 2> cl = ldpack<int32_t, 2>(a.col + k * a.ld + i0);
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const int64_t j = col_of(k, i0, r, cl);
+            const double gv = STORED ? (double)v1[j] : (double)iop_row<VT>(xs, c1, c0, qp[j], v1[j], v0[j]);
+            acc[r] = __fma_rn((double)w.v[r], gv, acc[r]);
+          }
+        }
+      }
+      if (i0 + 1 < n) {
+        stpair<double>(qn + i0, acc[0], acc[1]);
+        if constexpr (!STORED) stpair<VT>(vn + i0, (VT)x[0], (VT)x[1]);
+      } else {
+        qn[i0] = acc[0];
+        if constexpr (!STORED) vn[i0] = (VT)x[0];
+      }
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        if (i0 + r < n) {
+          iop_row_sums(x[r], STORED ? (c > 0 ? (double)l.o0.v[r] : 0.0) : (double)l.o1.v[r], acc[r], t);
+        }
+    }
+    iop_group_sums(t, p.part[c & 1], p.groups, g);
+  } else {
+    krylov_sink<VT, STORED>(a, p, (int)blockIdx.x - p.groups, v1, v0, vn, qp, qn);
+  }
+}
+
+template <typename VT, int K, int DM>
+void launch_col(bool stored, const LaunchCfg& c, const MatArgs<VT>& a, const IopArgs& p) {
+  auto k = stored ? k_krylov_col<VT, K, DM, true> : k_krylov_col<VT, K, DM, false>;
+  if (c.e0)
+    hipExtLaunchKernelGGL(k, dim3(c.grid), dim3(kIopThreads), 0, c.s, c.e0, c.e1, 0, a, p);
+  else
+    k<<<c.grid, kIopThreads, 0, c.s>>>(a, p);
+}
+
+template <typename VT, int DM>
+void dispatch_col_kd(bool stored, int K, const LaunchCfg& c, const MatArgs<VT>& a, const IopArgs& p) {
+  switch (K) {
+    case 1: launch_col<VT, 1, DM>(stored, c, a, p); break;
+    case 2: launch_col<VT, 2, DM>(stored, c, a, p); break;
+    case 3: launch_col<VT, 3, DM>(stored, c, a, p); break;
+    case 4: launch_col<VT, 4, DM>(stored, c, a, p); break;
+    case 5: launch_col<VT, 5, DM>(stored, c, a, p); break;
+    case 6: launch_col<VT, 6, DM>(stored, c, a, p); break;
+    case 7: launch_col<VT, 7, DM>(stored, c, a, p); break;
+    case 8: launch_col<VT, 8, DM>(stored, c, a, p); break;
+    default: launch_col<VT, 0, 2>(stored, c, a, p); break;
+  }
+}
+
+template <typename VT>
+void launch_krylov_t(nc_matrix_s* A, hipStream_t s, const IopArgs& p, hipEvent_t e0, hipEvent_t e1) {
+  const bool stored = p.c == 0;
+  const MatArgs<VT> a = mat_args<VT>(A, 0.0);
+  const LaunchCfg c{(unsigned)(p.groups + A->nr), s, e0, e1};
+  const uint32_t all = A->K >= 32 ? 0xffffffffu : ((1u << A->K) - 1u);
+  if (a.dia_mask == 0u)
+    dispatch_col_kd<VT, 0>(stored, A->K, c, a, p);
+  else if ((a.dia_mask & all) == all)
+    dispatch_col_kd<VT, 1>(stored, A->K, c, a, p);
+  else
+    launch_col<VT, 0, 2>(stored, c, a, p);
 }
 
 // ---- matrix-free setup --------------------------------------------------------------
@@ -1708,30 +1927,36 @@ void matvec_launch_err(nc_matrix_s* A, double t, const void* v, double* out, hip
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool timed = matvec_timing_slot(A, &e0, &e1);
   if (A->precision == NC_FP32)
-    launch_matvec_t<float>(A, t, v, out, false, s, true, e0, e1, nullptr, nullptr, &epi);
+    launch_matvec_t<float>(A, t, v, out, false, s, true, e0, e1, nullptr, &epi);
   else
-    launch_matvec_t<double>(A, t, v, out, false, s, true, e0, e1, nullptr, nullptr, &epi);
+    launch_matvec_t<double>(A, t, v, out, false, s, true, e0, e1, nullptr, &epi);
   NC_CHECK_HIP(hipGetLastError());
   if (timed) A->ev_used++;
   A->launches++;
 }
 
-bool matvec_dots_fusable(const nc_matrix_s* A) {
-  if (A->mf_mode != 0 || A->rows_per_thread != 2 || (A->timing && A->timing_plain) || !A->tv_r.empty() || A->K < 1 ||
-      A->K > 8)
-    return false;
-  const uint32_t all = (1u << A->K) - 1u;
-  return A->dia_mask == 0u || (A->dia_mask & all) == all;
+void krylov_form(const IopArgs& p, bool fp32, hipStream_t s) {
+  if (fp32)
+    launch_form<float>(p, s);
+  else
+    launch_form<double>(p, s);
 }
 
-void matvec_launch_dots(nc_matrix_s* A, const void* v, double* out, hipStream_t s, const DualDots& d) {
-  if (s != A->stream.s) throw Error(NC_ERR_INTERNAL, "projection mat-vec off the matrix stream");
+bool matvec_krylov_fusable(const nc_matrix_s* A) {
+  return A->mf_mode == 0 && A->rows_per_thread == 2 && !(A->timing && A->timing_plain) && A->tv_r.empty() &&
+         A->K >= 1 && A->n >= 1 && A->n_chunks == 0;
+}
+
+void matvec_launch_krylov(nc_matrix_s* A, hipStream_t s, const IopArgs& p) {
+  if (s != A->stream.s) throw Error(NC_ERR_INTERNAL, "Krylov column off the matrix stream");
+  if (!matvec_krylov_fusable(A) || p.n != A->n || p.tail1 != A->n_rows || A->n_rows > p.ld || A->nr > kIopTail)
+    throw Error(NC_ERR_INTERNAL, "Krylov column does not match the generator");
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool timed = matvec_timing_slot(A, &e0, &e1);
   if (A->precision == NC_FP32)
-    launch_matvec_t<float>(A, 0.0, v, out, false, s, true, e0, e1, nullptr, &d);
+    launch_krylov_t<float>(A, s, p, e0, e1);
   else
-    launch_matvec_t<double>(A, 0.0, v, out, false, s, true, e0, e1, nullptr, &d);
+    launch_krylov_t<double>(A, s, p, e0, e1);
   NC_CHECK_HIP(hipGetLastError());
   if (timed) A->ev_used++;
   A->launches++;
@@ -1824,9 +2049,9 @@ double bench_matvec(nc_matrix_s* A, double t, int reps) {
   return ms / reps;
 }
 
-// Mean duration of the mat-vec with the Krylov projection epilogue over nv basis vectors
-// (device-resident zero vectors in the solver's padded layout), launched reps times back
-// to back on the matrix's stream.
+// Mean duration of the Krylov process's column kernel at basis vector nv (device-resident
+// zero vectors in the solver's padded layout), launched reps times back to back on the
+// matrix's stream.
 double bench_projection(nc_matrix_s* A, int nv, int reps) {
   const bool was = A->timing, was_plain = A->timing_plain;
   A->timing = false;
@@ -1839,26 +2064,39 @@ double bench_projection(nc_matrix_s* A, int nv, int reps) {
       A->timing_plain = p;
     }
   } restore{A, was, was_plain};
-  if (!matvec_dots_fusable(A))
-    throw Error(NC_ERR_UNSUPPORTED, "this generator's mat-vec has no projection epilogue (it needs the stored "
-                                    "generator, 2 rows per thread, 1..8 slots, no time-varying reactions)");
+  if (!matvec_krylov_fusable(A))
+    throw Error(NC_ERR_UNSUPPORTED, "this generator's mat-vec has no Krylov column form (it needs the stored "
+                                    "generator, 2 rows per thread, short sink rows, no time-varying reactions)");
   NC_REQUIRE(nv >= 1 && nv <= 32, NC_ERR_ARG, "nv must be in 1..32");
-  const int64_t nblk = (A->n + kDualRows - 1) / kDualRows;
-  NC_REQUIRE(nblk >= 1 && nblk <= kDualMaxBlocks, NC_ERR_UNSUPPORTED, "state count outside the projection blocks' range");
   hipStream_t s = A->stream.s;
   const int64_t Np = (A->n_rows + 1023) / 1024 * 1024;
   DevBuf<unsigned char> V((size_t)nv * Np * A->vsize);
-  DevBuf<double> o(Np), part((size_t)(2 * nv + 1) * nblk);
+  IopArgs p{};
+  p.n = A->n;
+  p.tail1 = A->n_rows;
+  p.ld = Np;
+  p.nblk = (A->n + kIopRows - 1) / kIopRows;
+  p.groups = iop_groups(p.nblk);
+  p.c = nv - 1;
+  p.V = V.p;
+  p.L = KLayout{31};
+  p.btol = 1e-7;
+  DevBuf<double> q(2 * Np), part((size_t)2 * kIopSums * p.groups), kb(p.L.size_with_sinks(A->nr));
+  p.q[0] = q.p;
+  p.q[1] = q.p + Np;
+  p.part[0] = part.p;
+  p.part[1] = part.p + (size_t)kIopSums * p.groups;
+  p.kb = kb.p;
   NC_CHECK_HIP(hipMemsetAsync(V.p, 0, (size_t)nv * Np * A->vsize, s));
-  NC_CHECK_HIP(hipMemsetAsync(o.p, 0, sizeof(double) * Np, s));
-  const DualDots d{V.p, Np, nv, nullptr, part.p, nblk};
-  const void* vlast = V.p + (size_t)(nv - 1) * Np * A->vsize;
-  matvec_launch_dots(A, vlast, o.p, s, d);  // warm-up
+  NC_CHECK_HIP(hipMemsetAsync(q.p, 0, sizeof(double) * q.n, s));
+  NC_CHECK_HIP(hipMemsetAsync(part.p, 0, sizeof(double) * part.n, s));
+  NC_CHECK_HIP(hipMemsetAsync(kb.p, 0, sizeof(double) * kb.n, s));
+  matvec_launch_krylov(A, s, p);  // warm-up
   hipEvent_t e0, e1;
   NC_CHECK_HIP(hipEventCreate(&e0));
   NC_CHECK_HIP(hipEventCreate(&e1));
   NC_CHECK_HIP(hipEventRecord(e0, s));
-  for (int k = 0; k < reps; ++k) matvec_launch_dots(A, vlast, o.p, s, d);
+  for (int k = 0; k < reps; ++k) matvec_launch_krylov(A, s, p);
   NC_CHECK_HIP(hipEventRecord(e1, s));
   NC_CHECK_HIP(hipEventSynchronize(e1));
   float ms = 0.f;

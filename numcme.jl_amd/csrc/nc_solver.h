@@ -25,24 +25,21 @@ struct nc_solver_s {
   int32_t n_snaps = 0;
   // reduction scratch
   nc::DevBuf<double> partials;
-  nc::DevBuf<double> fold;  // folded totals of a vector pass and the fold's arrival counter
   unsigned red_blocks = 0;
-  int64_t dblk = 0;  // Krylov: 512-row projection blocks over the states (0: grid-stride passes)
+  int64_t kn = 0, kblk = 0;  // Krylov columns: rows summed in blocks, and the blocks
+  int kgroups = 0;           // their workgroups
   // Krylov
   int m = 30;
   nc::DevBuf<unsigned char> V;  // (m+1) x N, VT, unnormalised
-  nc::DevBuf<double> q;         // FP64 mat-vec output
-  nc::DevBuf<double> kbuf;      // H (m+2)^2 | h (m+2) | sc (m+2) | misc (8) | sink rows
-  nc::DevBuf<double> gram;      // (m+1)^2 Gram matrix of the scaled basis
-  nc::DevBuf<double> coef;      // combination coefficients (m+2)
-  double* hbuf = nullptr;       // pinned host copy of kbuf
-  double* hcoef = nullptr;      // pinned host staging of coef
+  nc::DevBuf<double> q;         // FP64 mat-vec outputs of two columns
+  nc::DevBuf<double> kbuf;      // H (m+2)^2 | sc (m+2) | misc (8) | sink rows
+  double* hbuf = nullptr;       // pinned host copy of kbuf, written by the process's last launch
+  double* hbuf_dev = nullptr;   // the same block as a device address
   double* hpart = nullptr;      // pinned host copy of per-block partial sums
   int64_t hpart_cap = 0;        // partial slots of hpart before its sink-value region
   double* hpart_dev = nullptr;  // the same pinned block as a device address: the RK error
                                 // pass writes its partials there directly
   double beta = 0.0, t_new = 0.0, anorm = 0.0;
-  bool beta_pending = false;  // beta was updated on the device and not yet read back
   bool started = false;
   hipGraph_t arnoldi_graph = nullptr;  // captured Arnoldi process (replayed every step)
   hipGraphExec_t arnoldi_exec = nullptr;
@@ -64,7 +61,6 @@ struct nc_solver_s {
     if (arnoldi_graph) (void)hipGraphDestroy(arnoldi_graph);
     if (s) (void)hipStreamSynchronize(s);  // copies into the pinned blocks have landed
     if (hbuf) nc::pinned_free(hbuf);
-    if (hcoef) nc::pinned_free(hcoef);
     if (hpart) nc::pinned_free(hpart);
   }
 };
@@ -87,5 +83,5 @@ void solver_set_state_device(nc_solver_s* S, double t0, const double* u_dev);
 double solver_step_hint(const nc_solver_s* S);
 // Start the next step from h instead of the automatic first step (h <= 0: no change).
 void solver_seed_step(nc_solver_s* S, double h);
-void solver_reduce_setup(nc_solver_s* S, int nvals);
+void solver_reduce_setup(nc_solver_s* S);
 }  // namespace nc

@@ -3,10 +3,9 @@
 // Replaces the integrator loop of NumCME.jl's solve (src/transientcme/sparse/fspsolve.jl:
 // 10-41, a DifferentialEquations.jl/CVODE call around matvec!) with:
 //
-//  * Krylov expv for time-invariant generators: Arnoldi by classical Gram-Schmidt whose
-//    coefficients solve the Gram system of the stored basis (one projection pass and one
-//    update pass per column, orthogonal to FP64 rounding even with an FP32 basis), FP64
-//    dot products and coefficients, basis vectors stored in the matrix precision; the
+//  * Krylov expv for time-invariant generators: incomplete orthogonalisation against the
+//    last two basis vectors (nc_iop.h), FP64 dot products and coefficients, basis vectors
+//    stored in the matrix precision, one launch per basis vector; the
 //    (m+2)x(m+2) Hessenberg exponential, the local error estimate and the step-size
 //    control run on the host, following R. B. Sidje, "Expokit: a software package for
 //    computing matrix exponentials", ACM TOMS 24(1), 1998 (algorithm of its EXPV
@@ -21,7 +20,6 @@
 #include <limits>
 #include <type_traits>
 
-#include "nc_dual.h"
 #include "nc_fspvec.h"
 #include "nc_solver.h"
 
@@ -31,326 +29,74 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kMaxRedBlocks = 2048;
-constexpr int kPartStrideMax = 65;  // partial sums per block: up to 2 x 32 dots + a norm
 
-// FIN_FOLD: the finish kernel only folds the partials into a.tot (the next pass, an
-// update with arn_pre set, applies the Arnoldi finishing step itself)
-enum Finish : int { FIN_NONE = 0, FIN_LAST, FIN_BETA, FIN_SUMS, FIN_FOLD };
-constexpr double kBreakdownTol = 1e-7;   // Expokit's happy-breakdown threshold
-// threads of each fold workgroup: one partial per thread at the 1,024-workgroup grid (a
-// thread looping over several would wait for each load in turn)
-constexpr int kFinBlock = 1024;
-constexpr unsigned kVecBlocks = 512;  // grid of the vector passes
+// Happy breakdown: the residual of the exhausted space is |beta| h per unit time, so h has to
+// fall below the tolerance the caller asks for, per unit time too (Expokit's fixed 1e-7
+// let a solve near its stationary state jump to the next output with 1e-6 of error).
+inline double breakdown_tol(const nc_solver_s* S) { return std::min(1e-7, std::max(1e-14, S->opts.krylov_tol)); }
+constexpr int kFinBlock = 1024;          // threads of the square-sum fold
+constexpr unsigned kVecBlocks = 512;     // grid of the vector passes
 constexpr int kLoadChunk = 8;  // basis vectors whose loads a vector pass issues together
-constexpr int kJacobiSweeps = 3;  // G h = a with G = I + O(1e-7): the error falls 1e-6 per sweep
-
-// kbuf layout (doubles)
-struct KLayout {
-  int m;
-  __host__ __device__ int H(int i, int j) const { return i * (m + 2) + j; }
-  __host__ __device__ int h(int i) const { return (m + 2) * (m + 2) + i; }
-  __host__ __device__ int sc(int i) const { return (m + 2) * (m + 2) + (m + 2) + i; }
-  __host__ __device__ int misc(int i) const { return (m + 2) * (m + 2) + 2 * (m + 2) + i; }
-  // sink rows of basis vector j (j <= m) and of the state (j = m+1), R sinks each
-  __host__ __device__ int sinkv(int j, int r, int R) const { return misc(8) + j * R + r; }
-  __host__ __device__ int size() const { return (m + 2) * (m + 2) + 2 * (m + 2) + 8; }
-  __host__ __device__ int size_with_sinks(int R) const { return size() + (m + 2) * R; }
-};
-enum { MISC_AVN = 0, MISC_BETA = 1 };
-
-template <typename BT>
-struct VecArgs {
-  int64_t N;
-  int nv;
-  const BT* V;            // nv x N basis (raw)
-  const double* sc;       // per-vector scale (device, may be null = 1)
-  const double* coef;     // per-vector coefficient (device, may be null)
-  double csign;           // multiplies coef
-  const double* xin;      // FP64 input
-  const double* xscale;   // device scalar multiplying xin (may be null = 1)
-  double* xout;           // FP64 outputs (nullable)
-  void* vout;             // VT output (nullable)
-  int vout_fp32;          // 1: vout is float, 0: double
-  int mode;               // VM_*
-  double* partials;
-  int finish;
-  double* kb;
-  double* gram;           // (m+1) x (m+1) Gram matrix of the scaled basis (arn_pre)
-  double* tot;            // kPartStrideMax folded totals (finish)
-  int arn_pre;            // VM_UPDATE: apply column j's Arnoldi finishing step from tot first
-  unsigned* counter;      // arrival counter of the fold's workgroups, zero between passes
-  KLayout L;
-  int j;
-  double btol;
-  int64_t tail0, tail1;   // fold: rows [tail0, tail1) of V and xin (the sink rows) added to the
-                          // block sums of the 512-row projection passes
-};
 
 __device__ inline double wave_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
   return v;
 }
 
-// Partial sums are stored value-major, partials[k * nblocks + b], so the finish kernel's
-// loads of one value across all blocks are contiguous.
-//
-// x = xscale*xin + csign * sum_i coef[i]*sc[i]*V_i, with optional FP64 / VT stores of x,
-// and per-block partial sums of what the pass measures:
-//   VM_DOTS    x = xscale*xin; d_i = sc[i] * sum_n V_i[n] x[n]        (nv dots)
-//   VM_UPDATE  the update, no dots
-//   VM_DUAL    x = xin; p_i = sum_n V_i[n] x[n] and g_i = sum_n V_i[n] V_last[n]
-//              with V_last = V_{nv-1}                                  (2 nv dots)
-// and always the norm sum_n x[n]^2 last. Each thread owns 4 consecutive rows and reads
-// every stream with one 16-byte (FP32) or 32-byte (FP64) vector load per vector; N is a
-// multiple of 4 and all vectors are zero beyond the true length, so no tail handling is
-// needed.
-enum VecMode : int { VM_DOTS = 0, VM_UPDATE = 1, VM_DUAL = 2 };
-
 template <typename T, int R>
 struct alignas(sizeof(T) * R) Pack {
   T v[R];
 };
 
-// Finishing step of Arnoldi column j from the folded totals tot (V_i.q at i, V_i.V_j at
-// nv + i, nv = j + 1), done by every workgroup of the update pass that follows instead of
-// by one workgroup in a launch of its own: |V_j| (H(j, j-1), sc_j), the Gram column of the
-// scaled basis, and h from G h = a, a_i = sc_i sc_j V_i.q, by Jacobi sweeps (G is the
-// identity up to the FP32 rounding of the stored basis). Leaves the update coefficients
-// -h_i sc_i in cs[0..nv) and sc_j in *xs; workgroup 0 also stores H(., j), h, sc_j and the
-// Gram column for the later columns (no other workgroup reads those entries). kBlock
-// threads: the sweeps give each row i eight lanes.
-__device__ void arnoldi_prologue(const KLayout& L, double* kb, double* gram, int j, double btol, const double* tot,
-                                 double* cs, double* xs) {
-  static_assert(kBlock == 256, "arnoldi_prologue assumes 256 threads");
-  const int nv = j + 1, ld = L.m + 1;
-  __shared__ double p_scj, p_nj, p_a[32], p_h[32], p_sc[32], p_tot[kPartStrideMax], p_G[32][33];
-  const int tid = threadIdx.x;
-  // every global read in one round trip: the previous Gram block, the scales, the totals
-  for (int e = tid; e < j * j; e += kBlock) p_G[e / j][e % j] = gram[(e / j) * ld + e % j];
-  if (tid < j || (j == 0 && tid == 0)) p_sc[tid] = kb[L.sc(tid)];  // sc(j), j >= 1, is set below
-  if (tid < 2 * nv) p_tot[tid] = tot[tid];
-  __syncthreads();
-  if (tid == 0) {
-    double nj = 0.0, scj = p_sc[0];
-    if (j >= 1) {
-      nj = sqrt(p_tot[nv + j]);
-      scj = nj > btol ? 1.0 / nj : 0.0;
-    }
-    p_nj = nj;
-    p_scj = scj;
-  }
-  __syncthreads();
-  const double scj = p_scj;
-  if (tid < nv) {
-    const int r = tid;
-    const double scr = r == j ? scj : p_sc[r];
-    double grj = scr * scj * p_tot[nv + r];
-    if (r == j && scj == 0.0) grj = 1.0;  // a vanished vector: keep G invertible
-    p_G[r][j] = grj;
-    p_G[j][r] = grj;
-    const double ar = scr * scj * p_tot[r];
-    p_a[r] = ar;
-    p_h[r] = ar;
-  }
-  if (tid == 0) p_sc[j] = scj;
-  __syncthreads();
-  const int i = tid >> 3, kq = tid & 7;
-  for (int sweep = 0; sweep < kJacobiSweeps; ++sweep) {
-    double t = 0.0;
-    if (i < nv)
-      for (int k = kq; k < nv; k += 8) t += (k == i ? p_G[i][k] - 1.0 : p_G[i][k]) * p_h[k];
-    for (int off = 4; off > 0; off >>= 1) t += __shfl_down(t, off, 8);
-    __syncthreads();
-    if (kq == 0 && i < nv) p_h[i] = p_a[i] - t;
-    __syncthreads();
-  }
-  if (tid < nv) cs[tid] = -p_h[tid] * p_sc[tid];
-  if (tid == 0) *xs = scj;
-  if (blockIdx.x == 0) {
-    if (tid == 0 && j >= 1) {
-      kb[L.H(j, j - 1)] = p_nj;
-      kb[L.sc(j)] = scj;
-    }
-    if (tid < nv) {
-      kb[L.H(tid, j)] = p_h[tid];
-      kb[L.h(tid)] = p_h[tid];
-      gram[tid * ld + j] = p_G[tid][j];
-      gram[j * ld + tid] = p_G[j][tid];
-    }
-  }
-}
+// The end of a Krylov step: u <- cu u + sum_i cs[i] V_{i+1} (the coefficients are kernel
+// arguments: no upload), with the next step's V_0 in storage precision. HBM / Infinity
+// Cache bound: every basis vector once.
+template <typename BT>
+struct CombineArgs {
+  int64_t N;
+  int nv;  // vectors V_1 .. V_nv
+  const BT* V1;
+  BT* v0;
+  double* u;
+  double cu;
+  double cs[32];
+};
 
-template <typename BT, int MAXV, int MODE>
-__global__ __launch_bounds__(kBlock) void k_vec(VecArgs<BT> a) {
-  constexpr int MV = MAXV > 0 ? MAXV : 1;
-  constexpr bool DOTS = MODE != VM_UPDATE;
-  constexpr bool UPD = MODE == VM_UPDATE;
-  constexpr bool DUAL = MODE == VM_DUAL;
+// Each thread owns 4 consecutive rows and reads every stream with one 16-byte (FP32) or
+// 32-byte (FP64) vector load per vector; N is a multiple of 4 and all vectors are zero
+// beyond the true length, so no tail handling is needed. The basis is read in chunks of
+// kLoadChunk vectors whose loads are issued together (unconditional, index clamped to
+// nv - 1: a guarded load becomes a branch that waits for it) and kept ahead of their
+// arithmetic by a scheduling barrier; left to itself the scheduler reuses one register set
+// and waits after every load. Vectors beyond nv carry a zero coefficient.
+template <typename BT, int MAXV>
+__global__ __launch_bounds__(kBlock) void k_combine(CombineArgs<BT> a) {
   constexpr int R = 4;
-  const int nv = a.nv;
-  // per-vector coefficients live in LDS (uniform broadcast reads)
-  __shared__ double s_cs[MV], s_sc[MV], s_xs;
-  if (threadIdx.x < MV) {
-    const int i = threadIdx.x;
-    const double sc = (i < nv) ? (a.sc ? a.sc[i] : 1.0) : 0.0;
-    s_sc[i] = sc;
-    s_cs[i] = (i < nv && a.coef) ? a.csign * a.coef[i] * sc : 0.0;
-  }
-  if (threadIdx.x == 0) s_xs = a.xscale ? *a.xscale : 1.0;
+  __shared__ double s_cs[32];
+  if (threadIdx.x < 32) s_cs[threadIdx.x] = (int)threadIdx.x < a.nv ? a.cs[threadIdx.x] : 0.0;
   __syncthreads();
-  const double xs = s_xs;
-  double dacc[DOTS ? MV : 1], gacc[DUAL ? MV : 1];
-#pragma unroll
-  for (int i = 0; i < (DOTS ? MV : 1); ++i) dacc[i] = 0.0;
-#pragma unroll
-  for (int i = 0; i < (DUAL ? MV : 1); ++i) gacc[i] = 0.0;
-  double nacc = 0.0;
   const int64_t groups = a.N / R;
   const int64_t stride = (int64_t)gridDim.x * kBlock;
   for (int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x; g < groups; g += stride) {
     const int64_t n0 = g * R;
     double x[R];
-    const Pack<double, R> xi = *reinterpret_cast<const Pack<double, R>*>(a.xin + n0);
-    Pack<BT, R> vl;
-    if constexpr (DUAL) vl = *reinterpret_cast<const Pack<BT, R>*>(a.V + (int64_t)(nv - 1) * a.N + n0);
+    const Pack<double, R> xi = *reinterpret_cast<const Pack<double, R>*>(a.u + n0);
     if constexpr (MAXV == 0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) x[r] = xs * xi.v[r];
+      for (int r = 0; r < R; ++r) x[r] = a.cu * xi.v[r];
     }
-    // The basis is read in chunks of kLoadChunk vectors whose loads are issued together
-    // (unconditional, index clamped to nv - 1: a guarded load becomes a branch that
-    // waits for it) and kept ahead of their arithmetic by a scheduling barrier; left to
-    // itself the scheduler reuses one register set and waits after every load, which
-    // streams the basis one vector at a time. Vectors beyond nv carry a zero coefficient
-    // (update) or land in dots that are never stored.
 #pragma unroll
     for (int i0 = 0; i0 < MAXV; i0 += kLoadChunk) {
       Pack<BT, R> vv[kLoadChunk];
 #pragma unroll
       for (int u = 0; u < kLoadChunk; ++u)
         if (i0 + u < MAXV)
-          vv[u] = *reinterpret_cast<const Pack<BT, R>*>(a.V + (int64_t)min(i0 + u, nv - 1) * a.N + n0);
+          vv[u] = *reinterpret_cast<const Pack<BT, R>*>(a.V1 + (int64_t)min(i0 + u, a.nv - 1) * a.N + n0);
       __builtin_amdgcn_sched_barrier(0);
       if (i0 == 0) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) x[r] = xs * xi.v[r];
+        for (int r = 0; r < R; ++r) x[r] = a.cu * xi.v[r];
       }
-#pragma unroll
-      for (int u = 0; u < kLoadChunk; ++u) {
-        const int i = i0 + u;
-        if (i >= MAXV) break;
-        if constexpr (UPD) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) x[r] += s_cs[i] * (double)vv[u].v[r];
-        } else {
-#pragma unroll
-          for (int r = 0; r < R; ++r) dacc[i] += (double)vv[u].v[r] * x[r];
-        }
-        if constexpr (DUAL) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) gacc[i] += (double)vv[u].v[r] * (double)vl.v[r];
-        }
-      }
-    }
-    if (a.xout) {
-      Pack<double, R> o;
-#pragma unroll
-      for (int r = 0; r < R; ++r) o.v[r] = x[r];
-      *reinterpret_cast<Pack<double, R>*>(a.xout + n0) = o;
-    }
-    if (a.vout) {
-      if (a.vout_fp32) {
-        Pack<float, R> o;
-#pragma unroll
-        for (int r = 0; r < R; ++r) o.v[r] = (float)x[r];
-        *reinterpret_cast<Pack<float, R>*>(reinterpret_cast<float*>(a.vout) + n0) = o;
-      } else {
-        Pack<double, R> o;
-#pragma unroll
-        for (int r = 0; r < R; ++r) o.v[r] = x[r];
-        *reinterpret_cast<Pack<double, R>*>(reinterpret_cast<double*>(a.vout) + n0) = o;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) nacc += x[r] * x[r];
-  }
-  if (a.finish == FIN_NONE) return;
-  // block reduction of the dots (scaled by sc[i] here) and the norm
-  __shared__ double red[2 * MV + 1][kBlock / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ndots = DOTS ? (DUAL ? 2 * nv : nv) : 0;
-  if constexpr (DOTS) {
-#pragma unroll
-    for (int i = 0; i < MAXV; ++i) {
-      if (i < nv) {
-        double v = wave_sum(dacc[i]) * s_sc[i];
-        if (lane == 0) red[i][wave] = v;
-        if constexpr (DUAL) {
-          double w = wave_sum(gacc[i]);
-          if (lane == 0) red[nv + i][wave] = w;
-        }
-      }
-    }
-  }
-  {
-    double v = wave_sum(nacc);
-    if (lane == 0) red[ndots][wave] = v;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x <= ndots) {
-    double s = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w) s += red[threadIdx.x][w];
-    a.partials[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
-  }
-  // k_vec_finish folds the partials in the next launch: the kernel boundary makes them
-  // visible across XCDs without a per-block L2 writeback fence
-}
-
-// The Arnoldi update V_{j+1} = sc_j q - sum_i h_i sc_i V_i with the column's finishing step
-// (arnoldi_prologue) in every workgroup. Each thread issues its first q rows and its first
-// kLoadChunk basis rows before the prologue (its barriers wait for LDS only, so the loads
-// stay in flight while it runs), which hides the prologue behind the streams.
-template <typename BT, int MAXV>
-__global__ __launch_bounds__(kBlock) void k_arn_update(VecArgs<BT> a) {
-  constexpr int R = 4, C0 = MAXV < kLoadChunk ? MAXV : kLoadChunk;
-  const int nv = a.nv;
-  const int64_t groups = a.N / R, stride = (int64_t)gridDim.x * kBlock;
-  int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int64_t gc = g < groups ? g : groups - 1;  // clamped: the loads are unconditional
-  Pack<double, R> xi = *reinterpret_cast<const Pack<double, R>*>(a.xin + gc * R);
-  Pack<BT, R> v0[C0];
-#pragma unroll
-  for (int u = 0; u < C0; ++u) v0[u] = *reinterpret_cast<const Pack<BT, R>*>(a.V + (int64_t)min(u, nv - 1) * a.N + gc * R);
-  __shared__ double s_cs[MAXV], s_xs;
-  if (threadIdx.x < MAXV) s_cs[threadIdx.x] = 0.0;
-  __syncthreads();
-  arnoldi_prologue(a.L, a.kb, a.gram, a.j, a.btol, a.tot, s_cs, &s_xs);
-  __syncthreads();
-  const double xs = s_xs;
-  BT* vout = reinterpret_cast<BT*>(a.vout);
-  for (; g < groups; g += stride) {
-    const int64_t n0 = g * R;
-    if (g != gc) {  // a later grid-stride row group (not prefetched)
-      xi = *reinterpret_cast<const Pack<double, R>*>(a.xin + n0);
-#pragma unroll
-      for (int u = 0; u < C0; ++u) v0[u] = *reinterpret_cast<const Pack<BT, R>*>(a.V + (int64_t)min(u, nv - 1) * a.N + n0);
-    }
-    double x[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) x[r] = xs * xi.v[r];
-#pragma unroll
-    for (int u = 0; u < C0; ++u) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) x[r] += s_cs[u] * (double)v0[u].v[r];
-    }
-#pragma unroll
-    for (int i0 = C0; i0 < MAXV; i0 += kLoadChunk) {
-      Pack<BT, R> vv[kLoadChunk];
-#pragma unroll
-      for (int u = 0; u < kLoadChunk; ++u)
-        if (i0 + u < MAXV)
-          vv[u] = *reinterpret_cast<const Pack<BT, R>*>(a.V + (int64_t)min(i0 + u, nv - 1) * a.N + n0);
-      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < kLoadChunk; ++u) {
         if (i0 + u >= MAXV) break;
@@ -358,293 +104,114 @@ __global__ __launch_bounds__(kBlock) void k_arn_update(VecArgs<BT> a) {
         for (int r = 0; r < R; ++r) x[r] += s_cs[i0 + u] * (double)vv[u].v[r];
       }
     }
-    Pack<BT, R> o;
+    Pack<double, R> o;
+    Pack<BT, R> ov;
 #pragma unroll
-    for (int r = 0; r < R; ++r) o.v[r] = (BT)x[r];
-    *reinterpret_cast<Pack<BT, R>*>(vout + n0) = o;
+    for (int r = 0; r < R; ++r) {
+      o.v[r] = x[r];
+      ov.v[r] = (BT)x[r];
+    }
+    *reinterpret_cast<Pack<double, R>*>(a.u + n0) = o;
+    *reinterpret_cast<Pack<BT, R>*>(a.v0 + n0) = ov;
   }
 }
 
-// VM_DUAL with the basis split across the workgroup's waves (wave w owns V_w, V_{w+4},
-// ...). Every wave streams the same rows of x and V_last, which the other waves' reads
-// keep in L2, and only its own basis vectors, so a thread holds 2 ceil(MAXV / 4)
-// accumulators instead of 2 MAXV and the pass keeps its occupancy at high column counts.
-// Same partial-sum layout as k_vec (each value is written by the wave that owns it).
-template <typename BT, int MAXV>
-__global__ __launch_bounds__(kBlock) void k_vec_dual(VecArgs<BT> a) {
-  constexpr int W = kBlock / 64, MVW = (MAXV + W - 1) / W, R = 4;
-  const int nv = a.nv;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const double xs = a.xscale ? *a.xscale : 1.0;
-  double dacc[MVW], gacc[MVW], nacc = 0.0;
-#pragma unroll
-  for (int k = 0; k < MVW; ++k) dacc[k] = gacc[k] = 0.0;
-  const BT* Vl = a.V + (int64_t)(nv - 1) * a.N;
-  const int64_t groups = a.N / R;
-  const int64_t stride = (int64_t)gridDim.x * 64;
-  for (int64_t g = (int64_t)blockIdx.x * 64 + lane; g < groups; g += stride) {
-    const int64_t n0 = g * R;
-    const Pack<double, R> xi = *reinterpret_cast<const Pack<double, R>*>(a.xin + n0);
-    const Pack<BT, R> vl = *reinterpret_cast<const Pack<BT, R>*>(Vl + n0);
-    // all of this wave's basis loads issued together (unconditional, clamped; see k_vec)
-    Pack<BT, R> vv[MVW];
-#pragma unroll
-    for (int k = 0; k < MVW; ++k)
-      vv[k] = *reinterpret_cast<const Pack<BT, R>*>(a.V + (int64_t)min(k * W + wave, nv - 1) * a.N + n0);
-    __builtin_amdgcn_sched_barrier(0);
-    double x[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) x[r] = xs * xi.v[r];
-#pragma unroll
-    for (int k = 0; k < MVW; ++k) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        dacc[k] += (double)vv[k].v[r] * x[r];
-        gacc[k] += (double)vv[k].v[r] * (double)vl.v[r];
-      }
-    }
-    if (wave == 0) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) nacc += x[r] * x[r];
-    }
-  }
-  const int64_t nb = gridDim.x;
-#pragma unroll
-  for (int k = 0; k < MVW; ++k) {
-    const int i = k * W + wave;
-    if (i < nv) {
-      const double d = wave_sum(dacc[k]) * (a.sc ? a.sc[i] : 1.0);
-      const double gm = wave_sum(gacc[k]);
-      if (lane == 0) {
-        a.partials[(int64_t)i * nb + blockIdx.x] = d;
-        a.partials[(int64_t)(nv + i) * nb + blockIdx.x] = gm;
-      }
-    }
-  }
-  if (wave == 0) {
-    const double v = wave_sum(nacc);
-    if (lane == 0) a.partials[(int64_t)(2 * nv) * nb + blockIdx.x] = v;
-  }
-}
-
-// Fold of the per-block partials, then the finishing step. One workgroup per value:
-// workgroup k sums value k over the pass's blocks in a fixed order (thread t takes blocks
-// t, t + 1024, ..., then a fixed shuffle tree), so the totals are deterministic, and
-// stores it. The workgroup that arrives last at a device-scope counter (release fence
-// before the increment, acquire fence after it) reads every total, re-arms the counter
-// for the next pass and applies the finishing step. The values are folded by nvals
-// compute units at once instead of one.
 template <typename BT>
-__global__ __launch_bounds__(kFinBlock) void k_vec_finish(VecArgs<BT> a, unsigned nblocks, int nvals) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __shared__ double tot[kPartStrideMax];
-  __shared__ double wsum[kFinBlock / 64];
-  __shared__ int s_last;
-  {
-    const int k = blockIdx.x;
-    // thread t takes blocks t, t + 1024, t + 2048, t + 3072 (nblocks <= 4096), loaded
-    // together and added in that order
-    double pv[4];
+void launch_combine(const CombineArgs<BT>& a, unsigned grid, hipStream_t s) {
+  switch ((a.nv + 7) / 8) {
+    case 0: k_combine<BT, 0><<<grid, kBlock, 0, s>>>(a); break;
+    case 1: k_combine<BT, 8><<<grid, kBlock, 0, s>>>(a); break;
+    case 2: k_combine<BT, 16><<<grid, kBlock, 0, s>>>(a); break;
+    case 3: k_combine<BT, 24><<<grid, kBlock, 0, s>>>(a); break;
+    default: k_combine<BT, 32><<<grid, kBlock, 0, s>>>(a); break;
+  }
+  NC_CHECK_HIP(hipGetLastError());
+}
+
+// Column c's five sums from the stored vectors, where the mat-vec does not form them (nc_iop.h)
+template <typename BT>
+__global__ __launch_bounds__(kIopThreads) void k_krylov_sums(IopArgs p) {
+  const int c = p.c, g = blockIdx.x;
+  const BT* V = reinterpret_cast<const BT*>(p.V);
+  const BT* __restrict__ v = V + (int64_t)c * p.ld;
+  const BT* __restrict__ v1 = V + (int64_t)(c > 0 ? c - 1 : 0) * p.ld;
+  const double* __restrict__ q = p.q[c & 1];
+  const int64_t blk0 = (int64_t)g * p.nblk / p.groups, blk1 = (int64_t)(g + 1) * p.nblk / p.groups;
+  double t[kIopSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int64_t blk = blk0; blk < blk1; ++blk) {
+    const int64_t i0 = blk * kIopRows + 2 * threadIdx.x;
+    if (i0 >= p.n) continue;
+    const Pack<double, 2> qv = *reinterpret_cast<const Pack<double, 2>*>(q + i0);
+    const Pack<BT, 2> a = *reinterpret_cast<const Pack<BT, 2>*>(v + i0), b = *reinterpret_cast<const Pack<BT, 2>*>(v1 + i0);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const unsigned b = threadIdx.x + u * kFinBlock;
-      const double t = a.partials[(int64_t)k * nblocks + min(b, nblocks - 1)];
-      pv[u] = b < nblocks ? t : 0.0;
-    }
-    double v = 0.0;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v += pv[u];
-    v = wave_sum(v);
-    if (lane == 0) wsum[wave] = v;
-    // the rows past the blocks (sink rows of the 512-row projection passes), by wave 0 in
-    // row order; value k is V_k.x (times sc_k), V_{k-nv}.V_{nv-1} or x.x as in the blocks
-    double tl = 0.0;
-    if (wave == 0 && a.tail1 > a.tail0) {
-      const int nv = a.nv;
-      const BT* Vl = a.V + (int64_t)(nv - 1) * a.N;
-      for (int64_t o = a.tail0 + lane; o < a.tail1; o += 64) {
-        const double xo = a.xin[o];
-        if (k < nv)
-          tl = __fma_rn((double)a.V[(int64_t)k * a.N + o], xo, tl);
-        else if (k < 2 * nv)
-          tl = __fma_rn((double)a.V[(int64_t)(k - nv) * a.N + o], (double)Vl[o], tl);
-        else
-          tl = __fma_rn(xo, xo, tl);
-      }
-      tl = wave_sum(tl);
-      if (k < nv && a.sc) tl *= a.sc[k];
-    }
-    __syncthreads();
-    if (a.finish == FIN_FOLD) {
-      // the totals are read by the next launch: its kernel boundary makes them visible
-      if (threadIdx.x == 0) {
-        double sum = 0.0;
-        for (int w = 0; w < kFinBlock / 64; ++w) sum += wsum[w];
-        a.tot[k] = sum + tl;
-      }
-      return;
-    }
-    if (threadIdx.x == 0) {
-      double sum = 0.0;
-      for (int w = 0; w < kFinBlock / 64; ++w) sum += wsum[w];
-      sum += tl;
-      __hip_atomic_store(reinterpret_cast<unsigned long long*>(a.tot) + k, (unsigned long long)__double_as_longlong(sum),
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __threadfence();
-      const unsigned prev = atomicAdd(a.counter, 1u);
-      const int last = prev + 1u == gridDim.x;
-      if (last) __threadfence();
-      s_last = last;
-    }
-    __syncthreads();
-    if (!s_last) return;
-    if ((int)threadIdx.x < nvals)
-      tot[threadIdx.x] = __longlong_as_double((long long)__hip_atomic_load(
-          reinterpret_cast<unsigned long long*>(a.tot) + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    if (threadIdx.x == 0) __hip_atomic_store(a.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int r = 0; r < 2; ++r)
+      if (i0 + r < p.n) iop_row_sums(a.v[r], c > 0 ? (double)b.v[r] : 0.0, qv.v[r], t);
+  }
+  iop_group_sums(t, p.part[c & 1], p.groups, g);
+}
+
+// The last column's norm and |A v_m| (avnorm of Expokit), the sink rows of the basis and of
+// the state u, and the step's coefficients to the pinned host block the host reads next (one
+// workgroup: no copy command, only the synchronisation).
+template <typename BT>
+__global__ __launch_bounds__(kIopThreads) void k_krylov_last(IopArgs p, int m, const double* u, int64_t ns, int R, double* host) {
+  double tot[kIopSums];
+  iop_fold<BT>(p, m, tot);
+  const IopCoef o = iop_coef(tot, m, 0.0, p.btol);  // the coefficients of V_{m+1} are not used
+  const KLayout L = p.L;
+  if (threadIdx.x == 0) {
+    p.kb[L.H(m, m - 1)] = o.nrm;
+    p.kb[L.sc(m)] = o.sc;
+    p.kb[L.misc(MISC_AVN)] = o.sc * sqrt(tot[4]);
+  }
+  const BT* V = reinterpret_cast<const BT*>(p.V);
+  for (int t = threadIdx.x; t < (m + 2) * R; t += kIopThreads) {
+    const int j = t / R, r = t % R;
+    host[L.sinkv(0, 0, R) + t] = j <= m ? (double)V[(int64_t)j * p.ld + ns + r] : u[ns + r];
   }
   __syncthreads();
-  const KLayout& L = a.L;
-  double* kb = a.kb;
+  for (int t = threadIdx.x; t < L.size(); t += kIopThreads) host[t] = p.kb[t];
+}
+
+// Sum of squares of x (N a multiple of 4) in two launches, deterministic.
+__global__ __launch_bounds__(kBlock) void k_sumsq(int64_t N, const double* x, double* part) {
+  double acc = 0.0;
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x; g < N / 4; g += stride) {
+    const Pack<double, 4> v = *reinterpret_cast<const Pack<double, 4>*>(x + 4 * g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc += v.v[r] * v.v[r];
+  }
+  __shared__ double red[kBlock / 64];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const double nrm2 = tot[nvals - 1];
-    switch (a.finish) {
-      case FIN_LAST: {
-        // VM_DUAL over V_m alone with x = A V_m: norm of V_m and |A v_m| for the error
-        // estimate (avnorm of Expokit)
-        const int m = L.m;
-        const double nm = sqrt(tot[1]);
-        const double scm = nm > a.btol ? 1.0 / nm : 0.0;
-        kb[L.H(m, m - 1)] = nm;
-        kb[L.sc(m)] = scm;
-        kb[L.misc(MISC_AVN)] = scm * sqrt(nrm2);
-      } break;
-      case FIN_BETA: {
-        const double b = sqrt(nrm2);
-        kb[L.misc(MISC_BETA)] = b;
-        kb[L.sc(0)] = b > 0.0 ? 1.0 / b : 0.0;
-      } break;
-      case FIN_SUMS:
-        for (int i = 0; i < nvals; ++i) kb[i] = tot[i];
-        break;
-      default: break;
-    }
+    double s = 0.0;
+    for (int w = 0; w < kBlock / 64; ++w) s += red[w];
+    part[blockIdx.x] = s;
   }
 }
 
-// The projection sums of Arnoldi column nv - 1 over 512-row blocks from the stored
-// q = A V_{nv-1} (nc_dual.h): the same block sums the mat-vec's projection epilogue forms,
-// for generators whose mat-vec has none. One workgroup per block.
-template <typename BT>
-__global__ __launch_bounds__(kBlock) void k_dual_blocks(const BT* __restrict__ V, int64_t ld, int nv,
-                                                        const double* __restrict__ q, int64_t n, double* part) {
-  const int64_t blk = blockIdx.x, base = blk * kDualRows;
-  const int lane = threadIdx.x & 63;
-  const BT* Vl = V + (int64_t)(nv - 1) * ld;
-  double x[8], y[8];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int64_t r = base + 256 * h + 4 * lane;
-    const Pack<double, 4> qx = *reinterpret_cast<const Pack<double, 4>*>(q + r);
-    const Pack<BT, 4> yl = *reinterpret_cast<const Pack<BT, 4>*>(Vl + r);
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const bool live = r + rr < n;
-      x[4 * h + rr] = live ? qx.v[rr] : 0.0;
-      y[4 * h + rr] = live ? (double)yl.v[rr] : 0.0;
-    }
+// one workgroup; nblocks <= kFinBlock
+__global__ __launch_bounds__(kFinBlock) void k_sumsq_fold(unsigned nblocks, const double* part, double* out) {
+  __shared__ double wsum[kFinBlock / 64];
+  const double v = wave_sum(threadIdx.x < nblocks ? part[threadIdx.x] : 0.0);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int w = 0; w < kFinBlock / 64; ++w) s += wsum[w];
+    *out = s;
   }
-  dual_block<BT>(V, ld, nv, base, x, y, nullptr, part, gridDim.x, blk);
 }
 
-template <typename BT, int MODE>
-void launch_vec_mode(const VecArgs<BT>& a, unsigned grid, hipStream_t s) {
-  const int nv = a.nv;
-  if (nv <= 0)
-    k_vec<BT, 0, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 4)
-    k_vec<BT, 4, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 8)
-    k_vec<BT, 8, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 12)
-    k_vec<BT, 12, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 16)
-    k_vec<BT, 16, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 20)
-    k_vec<BT, 20, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 24)
-    k_vec<BT, 24, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 28)
-    k_vec<BT, 28, MODE><<<grid, kBlock, 0, s>>>(a);
-  else if (nv <= 32)
-    k_vec<BT, 32, MODE><<<grid, kBlock, 0, s>>>(a);
-  else
-    throw Error(NC_ERR_UNSUPPORTED, "Krylov dimension above 31 is not supported");
-}
-
-template <typename BT>
-void launch_vec(VecArgs<BT> a, const nc_solver_s* S, hipStream_t s) {
-  if (a.N % 4) throw Error(NC_ERR_INTERNAL, "vector passes need a padded length");
-  if (!a.xin) throw Error(NC_ERR_INTERNAL, "vector passes need an input vector");
+// |x|^2 of a padded solver vector into *out (device)
+void launch_sumsq(const nc_solver_s* S, const double* x, double* out, hipStream_t s) {
   const unsigned grid = S->red_blocks;
-  a.tot = S->fold.p;
-  a.counter = reinterpret_cast<unsigned*>(S->fold.p + kPartStrideMax);
-  int nvals = 1;
-  switch (a.mode) {
-    case VM_DOTS: launch_vec_mode<BT, VM_DOTS>(a, grid, s); nvals = a.nv + 1; break;
-    case VM_DUAL:
-      nvals = 2 * a.nv + 1;
-      if (a.nv > 4 && a.nv <= 32 && !a.xout && !a.vout && a.finish != FIN_NONE) {
-        if (a.nv <= 8)
-          k_vec_dual<BT, 8><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 12)
-          k_vec_dual<BT, 12><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 16)
-          k_vec_dual<BT, 16><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 20)
-          k_vec_dual<BT, 20><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 24)
-          k_vec_dual<BT, 24><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 28)
-          k_vec_dual<BT, 28><<<grid, kBlock, 0, s>>>(a);
-        else
-          k_vec_dual<BT, 32><<<grid, kBlock, 0, s>>>(a);
-      } else {
-        launch_vec_mode<BT, VM_DUAL>(a, grid, s);
-      }
-      break;
-    default:
-      if (a.arn_pre) {
-        if (a.vout_fp32 != (std::is_same<BT, float>::value ? 1 : 0) || a.xout || !a.vout || a.finish != FIN_NONE)
-          throw Error(NC_ERR_INTERNAL, "Arnoldi update pass misconfigured");
-        if (a.nv <= 4)
-          k_arn_update<BT, 4><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 8)
-          k_arn_update<BT, 8><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 12)
-          k_arn_update<BT, 12><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 16)
-          k_arn_update<BT, 16><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 20)
-          k_arn_update<BT, 20><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 24)
-          k_arn_update<BT, 24><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 28)
-          k_arn_update<BT, 28><<<grid, kBlock, 0, s>>>(a);
-        else if (a.nv <= 32)
-          k_arn_update<BT, 32><<<grid, kBlock, 0, s>>>(a);
-        else
-          throw Error(NC_ERR_UNSUPPORTED, "Krylov dimension above 31 is not supported");
-      } else {
-        launch_vec_mode<BT, VM_UPDATE>(a, grid, s);
-      }
-      break;
-  }
-  if (a.finish != FIN_NONE) {
-    if (nvals > kPartStrideMax || !a.tot || !a.counter || grid > 4u * kFinBlock)
-      throw Error(NC_ERR_INTERNAL, "vector pass fold not set up");
-    k_vec_finish<BT><<<nvals, kFinBlock, 0, s>>>(a, grid, nvals);
-  }
+  if (S->Np % 4 || grid > (unsigned)kFinBlock) throw Error(NC_ERR_INTERNAL, "square sum not set up");
+  k_sumsq<<<grid, kBlock, 0, s>>>(S->Np, x, S->partials.p);
+  k_sumsq_fold<<<1, kFinBlock, 0, s>>>(grid, S->partials.p, out);
   NC_CHECK_HIP(hipGetLastError());
 }
 
@@ -768,18 +335,6 @@ __global__ __launch_bounds__(kBlock) void k_rk_hermite(int64_t N, double theta, 
     y[n] = a0 * y[n] + b0 * k0[n] + a1 * y1[n] + b1 * k6[n];
 }
 
-// Copy the sink rows (indices n_states .. n_states+R-1) of the m+1 basis vectors and of
-// the state u into the kbuf sink region, so the host can evaluate the sink-mass budget of
-// any combination of the basis.
-template <typename BT>
-__global__ void k_gather_sinks(const BT* V, int64_t ld, int nvec, const double* u, int64_t n_states, int R,
-                               double* dst) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (nvec + 1) * R) return;
-  const int j = t / R, r = t % R;
-  dst[t] = j < nvec ? (double)V[(int64_t)j * ld + n_states + r] : u[n_states + r];
-}
-
 __global__ void k_copy_d(const double* in, double* out, int64_t N) {
   const int64_t stride = (int64_t)gridDim.x * kBlock;
   for (int64_t n = (int64_t)blockIdx.x * kBlock + threadIdx.x; n < N; n += stride) out[n] = in[n];
@@ -800,28 +355,18 @@ double round_step(double x) {
 
 }  // namespace
 
-void solver_reduce_setup(nc_solver_s* S, int nvals) {
-  (void)nvals;
+void solver_reduce_setup(nc_solver_s* S) {
   // Grid of the vector passes: 1024 blocks of 256 threads for a Krylov basis stored in
   // FP32 and 512 otherwise (on the 1024^2 toggle-switch solve, 256 to 4096 blocks are
   // within 1% of each other since the passes issue their basis loads in batches)
   const unsigned vb = (S->method == NC_METHOD_KRYLOV && S->vs == 4) ? 1024u : kVecBlocks;
   S->red_blocks = std::min<unsigned>(vb, grid_for(S->Np / 4, kBlock));
-  // Krylov on one block: the projection sums go over 512-row blocks of the states (one
-  // workgroup each, the mat-vec's own row workgroups), folded with the sink rows
-  S->dblk = 0;
-  if (S->method == NC_METHOD_KRYLOV && !S->SA && S->blocks == 1) {
-    const int64_t nb = (S->A->n + kDualRows - 1) / kDualRows;
-    if (nb >= 1 && nb <= kDualMaxBlocks) S->dblk = nb;
-  }
-  // the RK error pass puts 3 R gathered sink values behind its partials
-  S->partials.reserve(std::max<size_t>({(size_t)S->red_blocks * kPartStrideMax, (size_t)S->dblk * kPartStrideMax,
-                                        (size_t)S->red_blocks + 3 * kMaxReactions}));
-  if (!S->fold.p) {
-    // folded totals, then the fold's arrival counter (zero between passes)
-    S->fold.alloc(kPartStrideMax + 1);
-    NC_CHECK_HIP(hipMemsetAsync(S->fold.p, 0, sizeof(double) * (kPartStrideMax + 1), S->s));
-  }
+  // Krylov columns: blocks of kIopRows state rows with the sink rows added by the fold; the
+  // sensitivity system sums every padded row
+  S->kn = S->SA ? S->Np : S->A->n;
+  S->kblk = std::max<int64_t>((S->kn + kIopRows - 1) / kIopRows, 1);
+  S->kgroups = iop_groups(S->kblk);
+  S->partials.reserve(std::max<size_t>(S->red_blocks, (size_t)2 * kIopSums * S->kgroups));
   if (!S->hpart) {
     // partials (up to kMaxRedBlocks, or one per row workgroup and sink row of the mat-vec's
     // error epilogue) and the RK step's 3 R gathered sink values, then the carried sinks of
@@ -858,152 +403,47 @@ static void copy_to_host(nc_solver_s* S, double* host, const double* dev) {
 }
 
 // ---- Krylov expv ---------------------------------------------------------------------
-// Arnoldi column j in two passes over the stored basis V_0..V_j (FP32 or FP64, kept
-// unnormalised with scales sc_i):
-//   pass 1 (VM_DUAL):   V_i.q and V_i.V_j for q = A V_j, folded into per-value totals
-//   pass 2 (VM_UPDATE): every workgroup first sets |V_j|, the Gram column of V_j and solves
-//                       G h = a, a_i = sc_i sc_j V_i.q, from the totals (arnoldi_prologue),
-//                       then V_{j+1} = sc_j q - sum_i h_i sc_i V_i
-// Projecting with the Gram matrix of the stored vectors makes V_{j+1} orthogonal to them
-// to FP64 rounding in one projection: the work a second classical Gram-Schmidt pass
-// would do, without a third pass over V.
-// q = A V_{nv-1} and the projection sums of V_0..V_{nv-1} (vbase) over 512-row blocks:
-// by the mat-vec's projection epilogue, or by the block pass over the stored q (the same
-// arithmetic), then folded with the sink rows by `finish`.
+// The device work of one Krylov process: columns 0 .. m (nc_iop.h), each one launch where
+// the generator's mat-vec has the column form, else V_c, q_c = A V_c and the sums by
+// themselves; then the last column's norms and the read-back. Its launches and arguments
+// are identical for every Krylov step, so it is captured once into a HIP graph and replayed.
 template <typename BT>
-static void dual_blocks_pass(nc_solver_s* S, const BT* vbase, int nv, int finish) {
-  nc_matrix_s* A = S->A;
-  const BT* vlast = vbase + (int64_t)(nv - 1) * S->Np;
-  if (matvec_dots_fusable(A)) {
-    const DualDots d{vbase, S->Np, nv, nullptr, S->partials.p, S->dblk};
-    matvec_launch_dots(A, vlast, S->q.p, S->s, d);
-  } else {
-    op_apply(S, 0.0, vlast, S->q.p);
-    k_dual_blocks<BT><<<(unsigned)S->dblk, kBlock, 0, S->s>>>(vbase, S->Np, nv, S->q.p, A->n, S->partials.p);
+static void krylov_process(nc_solver_s* S) {
+  IopArgs p{};
+  p.n = S->kn;
+  p.tail1 = S->SA ? S->kn : S->A->n_rows;
+  p.ld = S->Np;
+  p.nblk = S->kblk;
+  p.groups = S->kgroups;
+  p.V = S->V.p;
+  p.kb = S->kbuf.p;
+  p.L = KLayout{S->m};
+  p.btol = breakdown_tol(S);
+  for (int h = 0; h < 2; ++h) {
+    p.q[h] = S->q.p + (size_t)h * S->Np;
+    p.part[h] = S->partials.p + (size_t)h * kIopSums * S->kgroups;
+  }
+  const bool fused = !S->SA && matvec_krylov_fusable(S->A);
+  for (int c = 0; c <= S->m; ++c) {
+    p.c = c;
+    if (fused) {
+      matvec_launch_krylov(S->A, S->s, p);
+      continue;
+    }
+    if (c > 0) krylov_form(p, S->vs == 4, S->s);
+    op_apply(S, 0.0, S->V.p + (size_t)c * S->Np * S->vs, p.q[c & 1]);
+    k_krylov_sums<BT><<<(unsigned)S->kgroups, kIopThreads, 0, S->s>>>(p);
     NC_CHECK_HIP(hipGetLastError());
   }
-  VecArgs<BT> a{};
-  a.N = S->Np;
-  a.nv = nv;
-  a.V = vbase;
-  a.xin = S->q.p;
-  a.partials = S->partials.p;
-  a.kb = S->kbuf.p;
-  a.L = KLayout{S->m};
-  a.btol = kBreakdownTol;
-  a.finish = finish;
-  a.tot = S->fold.p;
-  a.counter = reinterpret_cast<unsigned*>(S->fold.p + kPartStrideMax);
-  a.tail0 = A->n;
-  a.tail1 = A->n + A->nr;
-  const int nvals = 2 * nv + 1;
-  if (nvals > kPartStrideMax || S->dblk > 4 * kFinBlock || a.tail1 > S->Np)
-    throw Error(NC_ERR_INTERNAL, "projection blocks not set up");
-  k_vec_finish<BT><<<nvals, kFinBlock, 0, S->s>>>(a, (unsigned)S->dblk, nvals);
+  k_krylov_last<BT><<<1, kIopThreads, 0, S->s>>>(p, S->m, S->u.p, S->A->n, S->A->nr, S->hbuf_dev);
   NC_CHECK_HIP(hipGetLastError());
 }
 
-template <typename BT>
-static void arnoldi_iteration(nc_solver_s* S, int j) {
-  const int64_t N = S->Np;
-  const KLayout L{S->m};
-  hipStream_t s = S->s;
-  auto Vp = [&](int i) { return reinterpret_cast<BT*>(S->V.p + (size_t)i * N * S->vs); };
-  if (S->dblk) {
-    dual_blocks_pass<BT>(S, Vp(0), j + 1, FIN_FOLD);
-    VecArgs<BT> a{};
-    a.N = N;
-    a.nv = j + 1;
-    a.V = Vp(0);
-    a.partials = S->partials.p;
-    a.kb = S->kbuf.p;
-    a.gram = S->gram.p;
-    a.L = L;
-    a.j = j;
-    a.btol = kBreakdownTol;
-    a.vout_fp32 = std::is_same<BT, float>::value ? 1 : 0;
-    a.xin = S->q.p;
-    a.mode = VM_UPDATE;
-    a.arn_pre = 1;
-    a.vout = Vp(j + 1);
-    a.finish = FIN_NONE;
-    launch_vec(a, S, s);
-    return;
-  }
-  op_apply(S, 0.0, Vp(j), S->q.p);
-  VecArgs<BT> a{};
-  a.N = N;
-  a.nv = j + 1;
-  a.V = Vp(0);
-  a.partials = S->partials.p;
-  a.kb = S->kbuf.p;
-  a.gram = S->gram.p;
-  a.L = L;
-  a.j = j;
-  a.btol = kBreakdownTol;
-  a.vout_fp32 = std::is_same<BT, float>::value ? 1 : 0;
-  a.mode = VM_DUAL;
-  a.xin = S->q.p;
-  a.finish = FIN_FOLD;
-  launch_vec(a, S, s);
-  // the update applies the finishing step (|V_j|, Gram column, h) from the folded totals
-  a.mode = VM_UPDATE;
-  a.arn_pre = 1;
-  a.vout = Vp(j + 1);
-  a.finish = FIN_NONE;
-  launch_vec(a, S, s);
-}
-
-template <typename BT>
-static void arnoldi_last(nc_solver_s* S) {
-  // |V_m| (H(m, m-1), sc_m) and avnorm = |A v_m| in one VM_DUAL pass over V_m
-  const KLayout L{S->m};
-  BT* vm = reinterpret_cast<BT*>(S->V.p + (size_t)S->m * S->Np * S->vs);
-  if (S->dblk) {
-    dual_blocks_pass<BT>(S, vm, 1, FIN_LAST);
-    return;
-  }
-  op_apply(S, 0.0, vm, S->q.p);
-  VecArgs<BT> a{};
-  a.N = S->Np;
-  a.nv = 1;
-  a.V = vm;
-  a.mode = VM_DUAL;
-  a.xin = S->q.p;
-  a.partials = S->partials.p;
-  a.kb = S->kbuf.p;
-  a.L = L;
-  a.btol = kBreakdownTol;
-  a.finish = FIN_LAST;
-  launch_vec(a, S, S->s);
-}
-
-// The device work of one Arnoldi process (m + 1 mat-vecs, the projections and the
-// |A v_m| norm). Its launches and arguments are identical for every Krylov step, so it is
-// captured once into a HIP graph and replayed.
 static void arnoldi_launch(nc_solver_s* S) {
-  const KLayout L{S->m};
-  const bool fp32 = S->A->precision == NC_FP32;
-  // V_0 (raw) and sc[0] = 1/beta are already on the device
-  for (int j = 0; j < S->m; ++j) {
-    if (fp32)
-      arnoldi_iteration<float>(S, j);
-    else
-      arnoldi_iteration<double>(S, j);
-  }
-  if (fp32)
-    arnoldi_last<float>(S);
+  if (S->A->precision == NC_FP32)
+    krylov_process<float>(S);
   else
-    arnoldi_last<double>(S);
-  const int R = S->A->nr;
-  double* dst = S->kbuf.p + L.sinkv(0, 0, R);
-  if (fp32)
-    k_gather_sinks<float><<<grid_for((int64_t)(S->m + 2) * R, kBlock), kBlock, 0, S->s>>>(reinterpret_cast<const float*>(S->V.p), S->Np, S->m + 1,
-                                                       S->u.p, S->A->n, R, dst);
-  else
-    k_gather_sinks<double><<<grid_for((int64_t)(S->m + 2) * R, kBlock), kBlock, 0, S->s>>>(reinterpret_cast<const double*>(S->V.p), S->Np, S->m + 1,
-                                                        S->u.p, S->A->n, R, dst);
-  NC_CHECK_HIP(hipGetLastError());
+    krylov_process<double>(S);
 }
 
 static void arnoldi_run(nc_solver_s* S) {
@@ -1081,9 +521,8 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
   hipStream_t s = S->s;
   const bool fp32 = A->precision == NC_FP32;
   const double tol = S->opts.krylov_tol;
-  const double btol = kBreakdownTol, gamma = 0.9, delta = 1.2;
+  const double btol = breakdown_tol(S), gamma = 0.9, delta = 1.2;
   const int mxrej = 10;
-  auto Vp = [&](int i) -> unsigned char* { return S->V.p + (size_t)i * N * S->vs; };
   if (!S->started) {
     // first step size from the norm estimate (Expokit)
     S->anorm = std::max(S->SA ? S->SA->norm1 : A->norm1, 1e-300);
@@ -1096,22 +535,18 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
   while (S->t < t_target - t_eps) {
     if (S->opts.max_steps && S->st.steps >= S->opts.max_steps)
       throw Error(NC_ERR_NUMERIC, "Krylov integrator exceeded max_steps");
-    if (S->beta == 0.0 && !S->beta_pending) {  // zero vector stays zero
+    if (S->beta == 0.0) {  // zero vector stays zero
       S->t = t_target;
       break;
     }
     double t_step = std::min(t_target - S->t, S->t_new);
     arnoldi_run(S);
     S->st.matvecs += m + 1;
-    NC_CHECK_HIP(hipMemcpyAsync(S->hbuf, S->kbuf.p, sizeof(double) * L.size_with_sinks(R), hipMemcpyDeviceToHost, s));
-    NC_CHECK_HIP(hipStreamSynchronize(s));
+    NC_CHECK_HIP(hipStreamSynchronize(s));  // the process ends by writing hbuf
     S->st.host_syncs++;
     matvec_harvest_timing(A);
     const double* hb = S->hbuf;
-    if (S->beta_pending) {
-      S->beta = hb[L.misc(MISC_BETA)];
-      S->beta_pending = false;
-    }
+    const double beta = hb[L.misc(MISC_BETA)];  // |V_0| as stored
     // happy breakdown detection
     int mb = m, k1 = 2;
     for (int j = 0; j < m; ++j) {
@@ -1142,8 +577,8 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
         err_loc = btol;
         break;
       }
-      const double phi1 = std::fabs(S->beta * F[m]);
-      const double phi2 = std::fabs(S->beta * F[m + 1] * avnorm);
+      const double phi1 = std::fabs(beta * F[m]);
+      const double phi2 = std::fabs(beta * F[m + 1] * avnorm);
       if (phi1 > 10.0 * phi2) {
         err_loc = phi2;
         xm = 1.0 / m;
@@ -1165,7 +600,7 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
       double tot = 0.0;
       for (int r = 0; r < R; ++r) {
         double v = Fm[0] * hb[L.sinkv(m + 1, r, R)];
-        for (int i = 1; i < mx; ++i) v += S->beta * Fm[i] * hb[L.sc(i)] * hb[L.sinkv(i, r, R)];
+        for (int i = 1; i < mx; ++i) v += beta * Fm[i] * hb[L.sc(i)] * hb[L.sinkv(i, r, R)];
         tot += v;
       }
       return tot;
@@ -1190,47 +625,25 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
       exp_tau(t_step, F);
       fire = true;
     }
-    // w_new = c0/beta * w + sum_{i>=1} c_i sc_i V_i ; c = beta * F[:,0]
-    double* coef = S->hcoef;  // pinned; the previous upload completed at the last sync
-    std::fill(coef, coef + m + 2, 0.0);
-    for (int i = 1; i < mx; ++i) coef[i - 1] = S->beta * F[i];
-    coef[m + 1] = F[0];  // (beta*F00)/beta
-    NC_CHECK_HIP(hipMemcpyAsync(S->coef.p, coef, sizeof(double) * (m + 2), hipMemcpyHostToDevice, s));
     S->t += t_step;
     const bool hit = !fire && S->t >= t_target - t_eps;
     if (hit) S->t = t_target;
-    {
-      auto fill = [&](auto& a, auto* vbase) {
-        a.N = N;
-        a.nv = mx - 1;
-        a.V = vbase;
-        a.sc = S->kbuf.p + L.sc(1);
-        a.coef = S->coef.p;
-        a.csign = 1.0;
-        a.xin = S->u.p;
-        a.xscale = S->coef.p + (m + 1);
-        a.xout = S->u.p;
-        a.vout = Vp(0);
-        a.vout_fp32 = fp32 ? 1 : 0;
-        a.partials = S->partials.p;
-        a.kb = S->kbuf.p;
-        a.L = L;
-        a.finish = FIN_BETA;
-        a.mode = VM_UPDATE;
-      };
-      if (fp32) {
-        VecArgs<float> a{};
-        fill(a, reinterpret_cast<const float*>(Vp(1)));
-        launch_vec(a, S, s);
-      } else {
-        VecArgs<double> a{};
-        fill(a, reinterpret_cast<const double*>(Vp(1)));
-        launch_vec(a, S, s);
-      }
-    }
-    // the new beta (written on the device by the combination) arrives with the next H
-    // download, so no synchronisation is needed here
-    S->beta_pending = true;
+    // w_new = F_0 w + sum_{i>=1} beta F_i sc_i V_i
+    auto combine = [&](auto* v0) {
+      CombineArgs<std::remove_pointer_t<decltype(v0)>> a{};
+      a.N = N;
+      a.nv = mx - 1;
+      a.V1 = v0 + N;
+      a.v0 = v0;
+      a.u = S->u.p;
+      a.cu = F[0];
+      for (int i = 1; i < mx; ++i) a.cs[i - 1] = (beta * F[i]) * hb[L.sc(i)];
+      launch_combine(a, S->red_blocks, s);
+    };
+    if (fp32)
+      combine(reinterpret_cast<float*>(S->V.p));
+    else
+      combine(reinterpret_cast<double*>(S->V.p));
     S->st.steps++;
     err_loc = std::max(err_loc, 1e-300);
     S->st.error_estimate += std::max(err_loc, S->anorm * 2.220446049250313e-16);
@@ -1332,19 +745,11 @@ void rk_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_step) {
   }
   if (S->h <= 0.0) {
     // initial step (Hairer, Norsett & Wanner, Solving ODEs I, II.4): based on |f(t0,y0)|
-    std::vector<double> sums(2);
-    VecArgs<double> a{};
-    a.N = N;
-    a.nv = 0;
-    a.xin = kp(0);
-    a.partials = S->partials.p;
-    a.kb = S->kbuf.p;
-    a.L = KLayout{S->m};
-    a.finish = FIN_SUMS;
-    launch_vec(a, S, s);
-    NC_CHECK_HIP(hipMemcpyAsync(sums.data(), S->kbuf.p, sizeof(double), hipMemcpyDeviceToHost, s));
+    double* fn2 = static_cast<double*>(host_stage(5));
+    launch_sumsq(S, kp(0), S->kbuf.p, s);
+    NC_CHECK_HIP(hipMemcpyAsync(fn2, S->kbuf.p, sizeof(double), hipMemcpyDeviceToHost, s));
     NC_CHECK_HIP(hipStreamSynchronize(s));
-    const double fnorm = std::sqrt(sums[0]);
+    const double fnorm = std::sqrt(*fn2);
     S->h = S->opts.h0 > 0 ? S->opts.h0 : (fnorm > 0 ? 0.01 / fnorm : 1e-3);
     S->h = std::max(S->h, 1e-12);
   }
@@ -1481,17 +886,14 @@ static nc_solver_s* solver_create_impl(nc_matrix_s* A, const nc_solve_opts* opts
       S->kbuf.alloc(ksize);
       NC_CHECK_HIP(hipMemsetAsync(S->kbuf.p, 0, sizeof(double) * ksize, S->s));
       S->hbuf = static_cast<double*>(pinned_alloc(sizeof(double) * ksize));
-      S->hcoef = static_cast<double*>(pinned_alloc(sizeof(double) * (S->m + 2)));
-      // k_vec writes partials with a stride of MAXV+1 <= 33 doubles per block
-      solver_reduce_setup(S, 32);
+      std::memset(S->hbuf, 0, sizeof(double) * ksize);
+      NC_CHECK_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&S->hbuf_dev), S->hbuf, 0));
+      solver_reduce_setup(S);
       if (method == NC_METHOD_KRYLOV) {
         S->V.alloc((size_t)(S->m + 1) * S->Np * S->vs);
-        S->q.alloc(S->Np);
+        S->q.alloc(2 * S->Np);  // columns alternate: a column gathers the last q while it writes its own
         NC_CHECK_HIP(hipMemsetAsync(S->V.p, 0, (size_t)(S->m + 1) * S->Np * S->vs, S->s));
-        NC_CHECK_HIP(hipMemsetAsync(S->q.p, 0, sizeof(double) * S->Np, S->s));
-        S->coef.alloc(S->m + 2);
-        S->gram.alloc((size_t)(S->m + 1) * (S->m + 1));
-        NC_CHECK_HIP(hipMemsetAsync(S->gram.p, 0, sizeof(double) * (S->m + 1) * (S->m + 1), S->s));
+        NC_CHECK_HIP(hipMemsetAsync(S->q.p, 0, sizeof(double) * 2 * S->Np, S->s));
       } else {
         S->rkv.alloc(S->Np * S->vs);
         S->k.alloc((size_t)7 * S->Np);
@@ -1524,10 +926,6 @@ static void solver_reinit(nc_solver_s* S) {
     S->st = nc_solve_stats{};
     if (S->method == NC_METHOD_KRYLOV) {
       S->beta = S->beta0;
-      S->beta_pending = false;
-      const KLayout L{S->m};
-      const double sc0 = S->beta > 0 ? 1.0 / S->beta : 0.0;
-      NC_CHECK_HIP(hipMemcpyAsync(S->kbuf.p + L.sc(0), &sc0, sizeof(double), hipMemcpyHostToDevice, S->s));
       const unsigned g = grid_for(S->Np, kBlock);
       if (S->A->precision == NC_FP32)
         k_to_vt<float><<<std::min(g, 4096u), kBlock, 0, S->s>>>(S->u.p, reinterpret_cast<float*>(S->V.p), S->Np);
@@ -1729,20 +1127,11 @@ void solver_set_state_device(nc_solver_s* S, double t0, const double* u_dev) {
   // u_dev holds the blocks contiguously (stride Nb); the solver pads each to Npb
   NC_CHECK_HIP(hipMemcpy2DAsync(S->u0.p, sizeof(double) * S->Npb, u_dev, sizeof(double) * S->Nb,
                                 sizeof(double) * S->Nb, S->blocks, hipMemcpyDeviceToDevice, S->s));
-  const KLayout L{S->m};
-  VecArgs<double> a{};
-  a.N = S->Np;
-  a.nv = 0;
-  a.xin = S->u0.p;
-  a.partials = S->partials.p;
-  a.kb = S->kbuf.p + L.misc(5);
-  a.L = L;
-  a.finish = FIN_SUMS;
-  launch_vec(a, S, S->s);
-  double b2 = 0.0;
-  NC_CHECK_HIP(hipMemcpyAsync(&b2, S->kbuf.p + L.misc(5), sizeof(double), hipMemcpyDeviceToHost, S->s));
+  double* b2 = static_cast<double*>(host_stage(5));
+  launch_sumsq(S, S->u0.p, S->kbuf.p, S->s);
+  NC_CHECK_HIP(hipMemcpyAsync(b2, S->kbuf.p, sizeof(double), hipMemcpyDeviceToHost, S->s));
   NC_CHECK_HIP(hipStreamSynchronize(S->s));
-  S->beta0 = std::sqrt(b2);
+  S->beta0 = std::sqrt(*b2);
   S->t0 = t0;
   solver_reinit(S);
   NC_CHECK_HIP(hipStreamSynchronize(S->s));
