@@ -72,6 +72,18 @@ struct EventSpec {
   double fsptol = 0.0, tend = 1.0;
   bool fired = false;
 };
+// The Krylov process of a small space in one launch (nc_krylov_small.hip): with nv >= 0 it
+// first ends the step before, u <- cu u + sum_{i < nv} cs[i] V_{i+1}. H, the scales, norms
+// and sink rows go to hbuf.
+bool krylov_small_fits(const nc_solver_s* S);
+void krylov_small_launch(nc_solver_s* S, int nv, double cu, const double* cs);
+// Happy breakdown: the residual of the exhausted space is |beta| h per unit time, so h has to
+// fall below the tolerance the caller asks for, per unit time too (Expokit's fixed 1e-7
+// let a solve near its stationary state jump to the next output with 1e-6 of error).
+inline double krylov_breakdown_tol(const nc_solver_s* S) {
+  const double tol = S->opts.krylov_tol;
+  return tol < 1e-14 ? 1e-14 : (tol < 1e-7 ? tol : 1e-7);
+}
 // Advance to t_target (or to the budget crossing when ev is given); with one_step the
 // call returns after the first accepted step.
 void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev = nullptr, bool one_step = false);

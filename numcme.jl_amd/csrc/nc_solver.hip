@@ -30,10 +30,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kMaxRedBlocks = 2048;
 
-// Happy breakdown: the residual of the exhausted space is |beta| h per unit time, so h has to
-// fall below the tolerance the caller asks for, per unit time too (Expokit's fixed 1e-7
-// let a solve near its stationary state jump to the next output with 1e-6 of error).
-inline double breakdown_tol(const nc_solver_s* S) { return std::min(1e-7, std::max(1e-14, S->opts.krylov_tol)); }
 constexpr int kFinBlock = 1024;          // threads of the square-sum fold
 constexpr unsigned kVecBlocks = 512;     // grid of the vector passes
 constexpr int kLoadChunk = 8;  // basis vectors whose loads a vector pass issues together
@@ -101,7 +97,7 @@ __global__ __launch_bounds__(kBlock) void k_combine(CombineArgs<BT> a) {
       for (int u = 0; u < kLoadChunk; ++u) {
         if (i0 + u >= MAXV) break;
 #pragma unroll
-        for (int r = 0; r < R; ++r) x[r] += s_cs[i0 + u] * (double)vv[u].v[r];
+        for (int r = 0; r < R; ++r) x[r] = __fma_rn(s_cs[i0 + u], (double)vv[u].v[r], x[r]);
       }
     }
     Pack<double, R> o;
@@ -418,7 +414,7 @@ static void krylov_process(nc_solver_s* S) {
   p.V = S->V.p;
   p.kb = S->kbuf.p;
   p.L = KLayout{S->m};
-  p.btol = breakdown_tol(S);
+  p.btol = krylov_breakdown_tol(S);
   for (int h = 0; h < 2; ++h) {
     p.q[h] = S->q.p + (size_t)h * S->Np;
     p.part[h] = S->partials.p + (size_t)h * kIopSums * S->kgroups;
@@ -521,7 +517,7 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
   hipStream_t s = S->s;
   const bool fp32 = A->precision == NC_FP32;
   const double tol = S->opts.krylov_tol;
-  const double btol = breakdown_tol(S), gamma = 0.9, delta = 1.2;
+  const double btol = krylov_breakdown_tol(S), gamma = 0.9, delta = 1.2;
   const int mxrej = 10;
   if (!S->started) {
     // first step size from the norm estimate (Expokit)
@@ -532,15 +528,46 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
     S->started = true;
   }
   const double t_eps = 1e-13 * std::max(1.0, std::fabs(t_target));
+  // the combination that ends a step: u <- pend_cu u + sum_i pend[i] V_{i+1}. A small space's
+  // next process takes it with it; else, and after the last step here, it is a launch.
+  const bool small = krylov_small_fits(S);
+  bool pending = false;
+  std::vector<double> pend;
+  double pend_cu = 0.0;
+  auto combine = [&](auto* v0) {
+    CombineArgs<std::remove_pointer_t<decltype(v0)>> a{};
+    a.N = N;
+    a.nv = (int)pend.size();
+    a.V1 = v0 + N;
+    a.v0 = v0;
+    a.u = S->u.p;
+    a.cu = pend_cu;
+    std::copy(pend.begin(), pend.end(), a.cs);
+    launch_combine(a, S->red_blocks, s);
+  };
+  auto end_step = [&] {
+    if (fp32)
+      combine(reinterpret_cast<float*>(S->V.p));
+    else
+      combine(reinterpret_cast<double*>(S->V.p));
+    pending = false;
+  };
   while (S->t < t_target - t_eps) {
-    if (S->opts.max_steps && S->st.steps >= S->opts.max_steps)
+    if (S->opts.max_steps && S->st.steps >= S->opts.max_steps) {
+      if (pending) end_step();
       throw Error(NC_ERR_NUMERIC, "Krylov integrator exceeded max_steps");
+    }
     if (S->beta == 0.0) {  // zero vector stays zero
       S->t = t_target;
       break;
     }
     double t_step = std::min(t_target - S->t, S->t_new);
-    arnoldi_run(S);
+    if (small) {
+      krylov_small_launch(S, pending ? (int)pend.size() : -1, pend_cu, pend.data());
+      pending = false;
+    } else {
+      arnoldi_run(S);
+    }
     S->st.matvecs += m + 1;
     NC_CHECK_HIP(hipStreamSynchronize(s));  // the process ends by writing hbuf
     S->st.host_syncs++;
@@ -629,21 +656,11 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
     const bool hit = !fire && S->t >= t_target - t_eps;
     if (hit) S->t = t_target;
     // w_new = F_0 w + sum_{i>=1} beta F_i sc_i V_i
-    auto combine = [&](auto* v0) {
-      CombineArgs<std::remove_pointer_t<decltype(v0)>> a{};
-      a.N = N;
-      a.nv = mx - 1;
-      a.V1 = v0 + N;
-      a.v0 = v0;
-      a.u = S->u.p;
-      a.cu = F[0];
-      for (int i = 1; i < mx; ++i) a.cs[i - 1] = (beta * F[i]) * hb[L.sc(i)];
-      launch_combine(a, S->red_blocks, s);
-    };
-    if (fp32)
-      combine(reinterpret_cast<float*>(S->V.p));
-    else
-      combine(reinterpret_cast<double*>(S->V.p));
+    pend_cu = F[0];
+    pend.resize(mx - 1);
+    for (int i = 1; i < mx; ++i) pend[i - 1] = (beta * F[i]) * hb[L.sc(i)];
+    pending = true;
+    if (!small || fire || hit || one_step) end_step();
     S->st.steps++;
     err_loc = std::max(err_loc, 1e-300);
     S->st.error_estimate += std::max(err_loc, S->anorm * 2.220446049250313e-16);
