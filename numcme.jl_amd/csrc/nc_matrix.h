@@ -71,7 +71,13 @@ struct nc_matrix_s {
   nc::DevBuf<int32_t> states;      // kept for joint refreshes
   nc::DevBuf<int32_t> state_conn;  // kept for joint refreshes
   nc_model_s* model = nullptr;     // borrowed; must outlive the matrix
-  double t_cache = -INFINITY;
+  double t_cache = -INFINITY;      // time of the joint values in tvd, tvv and sink_val
+  // further sets of those three arrays, each at a time of its own (matrix_prepare_times)
+  struct JointSet {
+    double t = -INFINITY;
+    nc::DevBuf<unsigned char> tvd, tvv, sink_val;
+  };
+  std::vector<JointSet> joint_sets;
   nc::Stream stream;
   // reporting
   int64_t nnz_ref = 0, n_sink_entries = 0;
@@ -95,6 +101,10 @@ constexpr size_t kNoAllocScratchBytes = size_t(48) << 20;
 nc_matrix_s* matrix_create(nc_space_s* sp, nc_model_s* m, int precision);
 // Bring time-dependent values up to date for time t (joint refresh, on the matrix stream).
 void matrix_prepare(nc_matrix_s* A, double t);
+// Joint values at several times to come (the stage times of an integrator step) by one
+// launch; mat-vecs at those times then find them. Nothing to do without joint reactions, and
+// above 2^18 states, where mat-vecs refresh at their own time.
+void matrix_prepare_times(nc_matrix_s* A, int count, const double* t);
 // Launch-time scales at t: sink rows (nr) and time-varying slots (tv_r.size()).
 void matrix_scales(const nc_matrix_s* A, double t, double* sink_scale, double* tv_scale);
 // out = A(t) v (+ out when accumulate); v is a device vector of n_rows VT values, out holds

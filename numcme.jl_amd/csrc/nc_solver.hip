@@ -704,6 +704,11 @@ void rk_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_step) {
   const bool efuse = fuse && !S->SA && err_parts <= S->hpart_cap;
   const int Rg = (ev && R > 0) ? R : 0;
   auto stages = [&](double h) {
+    if (!S->SA) {
+      double ts[5];
+      for (int j = 0; j < 5; ++j) ts[j] = S->t + h_dp_c[j + 1] * h;  // the last two stages share theirs
+      matrix_prepare_times(A, 5, ts);
+    }
     unsigned char* cur = S->rkv.p;
     unsigned char* nxt = S->rkv2.p;
     for (int stage = 1; stage < 7; ++stage) {
