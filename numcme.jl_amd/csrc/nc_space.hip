@@ -14,6 +14,7 @@
 //  * deleteat! (:276-331) is a keep-flag scan, a compaction with index remapping, a hash
 //    rebuild and a sink recomputation.
 #include <atomic>
+#include <type_traits>
 
 #include "nc_space.h"
 
@@ -67,46 +68,114 @@ __global__ void k_gen_candidates(const int32_t* states, const int32_t* stoich, i
   for (int s = 0; s < ns; ++s) cands[pos * ns + s] = states[src * ns + s] + stoich[s + r * ns];
 }
 
+// A state's counts in registers: NS is at least the species count, so the loops unroll (a
+// runtime count would put the array in scratch memory).
+template <int NS>
+struct Row {
+  int32_t x[NS];
+};
+template <int NS>
+__device__ inline Row<NS> load_row(const int32_t* p, int ns) {
+  Row<NS> r;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) r.x[s] = s < ns ? p[s] : 0;
+  return r;
+}
+template <int NS>
+__device__ inline bool row_nonneg(const Row<NS>& a) {
+  bool ok = true;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) ok = ok && a.x[s] >= 0;
+  return ok;
+}
+template <int NS>
+__device__ inline bool row_eq(const Row<NS>& a, const Row<NS>& b) {
+  bool eq = true;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) eq = eq && a.x[s] == b.x[s];
+  return eq;
+}
+template <int NS>
+__device__ inline uint64_t row_hash(const Row<NS>& a, int ns) {  // hash_state
+  uint64_t h = 0x9E3779B97F4A7C15ull * (uint64_t)(ns + 1);
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    if (s < ns) h = mix64(h ^ (uint64_t)(uint32_t)a.x[s]);
+  return h;
+}
+template <int NS, int SCOPE>
+__device__ inline int32_t row_find(const uint32_t* table, uint64_t mask, const int32_t* states, int ns,
+                                   const Row<NS>& x) {  // ht_find
+  uint64_t h = row_hash<NS>(x, ns) & mask;
+  for (;;) {
+    const uint32_t v = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, SCOPE);
+    if (v == HT_EMPTY) return -1;
+    if (!(v & HT_CAND) && row_eq<NS>(load_row<NS>(states + (int64_t)v * ns, ns), x)) return (int32_t)v;
+    h = (h + 1) & mask;
+  }
+}
+// Claim the slot of candidate `pos` with key x: its index, or -1 when x is in the space.
+// Every tag ever stored in a slot belongs to the same key, so comparing against the one read
+// is enough even if a smaller position replaces it concurrently. cand(p) is candidate p's key.
+template <int NS, int SCOPE, class CAND>
+__device__ inline int32_t row_claim(uint32_t* table, uint64_t mask, const int32_t* states, int ns, const Row<NS>& x,
+                                    uint32_t pos, CAND cand) {
+  const uint32_t tag = HT_CAND | pos;
+  uint64_t h = row_hash<NS>(x, ns) & mask;
+  for (;;) {
+    uint32_t v = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, SCOPE);
+    if (v == HT_EMPTY) {
+      uint32_t want = HT_EMPTY;
+      if (__hip_atomic_compare_exchange_strong(&table[h], &want, tag, __ATOMIC_RELAXED, __ATOMIC_RELAXED, SCOPE))
+        return (int32_t)h;
+      v = want;
+    }
+    if (v & HT_CAND) {
+      if (row_eq<NS>(cand(v & ~HT_CAND), x)) {
+        __hip_atomic_fetch_min(&table[h], tag, __ATOMIC_RELAXED, SCOPE);
+        return (int32_t)h;
+      }
+    } else if (row_eq<NS>(load_row<NS>(states + (int64_t)v * ns, ns), x)) {
+      return -1;
+    }
+    h = (h + 1) & mask;
+  }
+}
+// Connectivity of state idx along reaction r (sparsestatespace.jl:241-266)
+template <int NS, int SCOPE>
+__device__ inline void row_connect(const uint32_t* table, uint64_t mask, const int32_t* states, const int32_t* stoich,
+                                   int ns, int nr, int64_t idx, int r, int32_t* state_conn, uint32_t* sink_mask) {
+  const Row<NS> x = load_row<NS>(states + idx * ns, ns), d = load_row<NS>(stoich + r * ns, ns);
+  Row<NS> y, z;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) y.x[s] = x.x[s] - d.x[s], z.x[s] = x.x[s] + d.x[s];
+  if (row_nonneg<NS>(y)) {
+    const int32_t j = row_find<NS, SCOPE>(table, mask, states, ns, y);
+    if (j >= 0) {
+      state_conn[idx * nr + r] = j;
+      __hip_atomic_fetch_and(&sink_mask[j], ~(1u << r), __ATOMIC_RELAXED, SCOPE);
+    }
+  }
+  if (row_nonneg<NS>(z)) {
+    const int32_t k = row_find<NS, SCOPE>(table, mask, states, ns, z);
+    if (k < 0)
+      __hip_atomic_fetch_or(&sink_mask[idx], 1u << r, __ATOMIC_RELAXED, SCOPE);
+    else
+      state_conn[(int64_t)k * nr + r] = (int32_t)idx;
+  }
+}
+
+template <int NS>
 __global__ void k_cand_insert(uint32_t* table, uint64_t mask, const int32_t* states, const int32_t* cands, int ns,
                               int64_t n_cand, int32_t* slot_of) {
   int64_t pos = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (pos >= n_cand) return;
-  int32_t x[kMaxSpecies];
-  bool ok = true;
-  for (int s = 0; s < ns; ++s) {
-    x[s] = cands[pos * ns + s];
-    ok = ok && (x[s] >= 0);
-  }
-  if (!ok) {  // _is_all_nonnegative (sparsestatespace.jl:197-202)
-    slot_of[pos] = -1;
-    return;
-  }
-  const uint32_t tag = HT_CAND | (uint32_t)pos;
-  uint64_t h = hash_state(x, ns) & mask;
-  for (;;) {
-    uint32_t v = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (v == HT_EMPTY) {
-      uint32_t old = atomicCAS(&table[h], HT_EMPTY, tag);
-      if (old == HT_EMPTY) {
-        slot_of[pos] = (int32_t)h;
-        return;
-      }
-      v = old;
-    }
-    if (v & HT_CAND) {
-      // every tag ever stored in this slot belongs to the same key, so comparing against
-      // the one read is enough even if a smaller position replaces it concurrently
-      if (state_eq(cands + (int64_t)(v & ~HT_CAND) * ns, x, ns)) {
-        atomicMin(&table[h], tag);
-        slot_of[pos] = (int32_t)h;
-        return;
-      }
-    } else if (state_eq(states + (int64_t)v * ns, x, ns)) {
-      slot_of[pos] = -1;  // already in the space
-      return;
-    }
-    h = (h + 1) & mask;
-  }
+  const Row<NS> x = load_row<NS>(cands + pos * ns, ns);
+  // _is_all_nonnegative (sparsestatespace.jl:197-202)
+  slot_of[pos] = !row_nonneg<NS>(x) ? -1
+                                    : row_claim<NS, __HIP_MEMORY_SCOPE_AGENT>(
+                                          table, mask, states, ns, x, (uint32_t)pos,
+                                          [&](uint32_t p) { return load_row<NS>(cands + (int64_t)p * ns, ns); });
 }
 
 __global__ void k_first_flags(const uint32_t* table, const int32_t* slot_of, int64_t n_cand, uint32_t* flags) {
@@ -128,36 +197,149 @@ __global__ void k_commit(uint32_t* table, const int32_t* slot_of, const uint32_t
   table[slot_of[pos]] = (uint32_t)idx;
 }
 
-// Connectivity of the states [n_old, n_new): sparsestatespace.jl:241-266.
+// Connectivity of the states [n_old, n_new).
+template <int NS>
 __global__ void k_connect_new(const uint32_t* table, uint64_t mask, const int32_t* states, const int32_t* stoich,
                               int ns, int nr, int64_t n_old, int64_t n_new, int32_t* state_conn,
                               uint32_t* sink_mask) {
   int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (t >= (n_new - n_old) * nr) return;
-  int64_t idx = n_old + t / nr;
-  int r = (int)(t % nr);
-  int32_t y[kMaxSpecies], z[kMaxSpecies];
-  bool yok = true, zok = true;
-  for (int s = 0; s < ns; ++s) {
-    int32_t xs = states[idx * ns + s], d = stoich[s + r * ns];
-    y[s] = xs - d;
-    z[s] = xs + d;
-    yok = yok && y[s] >= 0;
-    zok = zok && z[s] >= 0;
+  row_connect<NS, __HIP_MEMORY_SCOPE_AGENT>(table, mask, states, stoich, ns, nr, n_old + t / nr, (int)(t % nr),
+                                            state_conn, sink_mask);
+}
+
+// ---- levels with few candidates ---------------------------------------------------------
+// A level of expansion is seven dependent launches and a synchronisation, 73 us however
+// small it is. While a level has at most kSmallCands candidates, one workgroup runs level
+// after level itself: the same passes separated by barriers, every atomic and every read
+// of the table and the sink masks at workgroup scope. It stops when a level would have
+// more, or when the rows or the table might not hold it, and says where.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallCands = 4096;
+constexpr int kSmallPer = kSmallCands / kSmallThreads;
+constexpr int64_t kSmallStates = int64_t(1) << 22;  // larger spaces are not grown for a few candidates
+struct ExpandArgs {
+  uint32_t* table;
+  uint64_t mask;
+  int32_t *states, *conn;
+  uint32_t* sinks;
+  const int32_t* stoich;
+  int32_t* list;           // the first level's explorables: written here first when n_flag >= 0
+  const uint32_t* select;  // flags, or null
+  int32_t ns, nr, levels;
+  uint32_t rmask;
+  int32_t n_flag;  // >= 0: find the explorables among this many states (at most kSmallCands)
+  int64_t n, base, nE, max_rows;
+  RList rl;
+  int64_t* out;  // pinned: levels done, states, first explorable, explorables, 1 if they are the list's
+};
+
+// Exclusive prefix sum over the workgroup in thread order, and the total; two barriers.
+__device__ inline int small_scan(int v, int* s_wave, int* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int inc = v;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += o;
   }
-  if (yok) {
-    int32_t j = ht_find(table, mask, states, ns, y);
-    if (j >= 0) {
-      state_conn[idx * nr + r] = j;
-      atomicAnd(&sink_mask[j], ~(1u << r));
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  int before = 0, all = 0;
+  for (int w = 0; w < kSmallThreads / 64; ++w) {
+    const int x = s_wave[w];
+    if (w < wave) before += x;
+    all += x;
+  }
+  __syncthreads();
+  *total = all;
+  return before + inc - v;
+}
+
+template <int NS>
+__global__ __launch_bounds__(kSmallThreads) void k_expand_small(ExpandArgs a) {
+  constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
+  __shared__ int s_wave[kSmallThreads / 64];
+  const int tid = threadIdx.x, ns = a.ns, nr = a.nr;
+  int64_t n = a.n, base = a.base, nE = a.nE;
+  const int32_t* list = a.list;
+  if (a.n_flag >= 0) {
+    int cnt = 0;
+    uint32_t f = 0;
+    for (int u = 0; u < kSmallPer; ++u) {
+      const int i = tid * kSmallPer + u;
+      if (i < a.n_flag && (a.sinks[i] & a.rmask) && (!a.select || a.select[i])) f |= 1u << u, ++cnt;
     }
+    int total;
+    int rank = small_scan(cnt, s_wave, &total);
+    for (int u = 0; u < kSmallPer; ++u)
+      if ((f >> u) & 1u) a.list[rank++] = tid * kSmallPer + u;
+    nE = total;
+    __syncthreads();
   }
-  if (zok) {
-    int32_t k = ht_find(table, mask, states, ns, z);
-    if (k < 0)
-      atomicOr(&sink_mask[idx], 1u << r);
-    else
-      state_conn[(int64_t)k * nr + r] = (int32_t)idx;
+  int level = 0;
+  for (; level < a.levels; ++level) {
+    const int64_t n_cand = nE * a.rl.n;
+    if (n_cand == 0 || n_cand > kSmallCands || n + n_cand > a.max_rows) break;
+    // candidate pos: explorable nE - 1 - pos / |R'| (last first), reaction R'[pos % |R'|]
+    auto cand = [&](uint32_t pos) {
+      const int64_t e = nE - 1 - pos / a.rl.n;
+      const Row<NS> x = load_row<NS>(a.states + (list ? (int64_t)list[e] : base + e) * ns, ns),
+                    d = load_row<NS>(a.stoich + a.rl.r[pos % a.rl.n] * ns, ns);
+      Row<NS> y;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) y.x[s] = x.x[s] + d.x[s];
+      return y;
+    };
+    const int per = (int)((n_cand + kSmallThreads - 1) / kSmallThreads);
+    int32_t slot[kSmallPer];
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+      slot[u] = -1;
+      const int pos = tid * per + u;
+      if (u < per && pos < n_cand) {
+        const Row<NS> x = cand(pos);
+        if (row_nonneg<NS>(x)) slot[u] = row_claim<NS, WG>(a.table, a.mask, a.states, ns, x, pos, cand);
+      }
+    }
+    __syncthreads();
+    int cnt = 0;
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+      // the slot's first occurrence keeps it
+      if (slot[u] >= 0 && __hip_atomic_load(&a.table[slot[u]], __ATOMIC_RELAXED, WG) != (HT_CAND | (uint32_t)(tid * per + u)))
+        slot[u] = -1;
+      cnt += slot[u] >= 0;
+    }
+    int added;
+    int64_t idx = n + small_scan(cnt, s_wave, &added);
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+      if (slot[u] < 0) continue;
+      const Row<NS> x = cand(tid * per + u);
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        if (s < ns) a.states[idx * ns + s] = x.x[s];
+      for (int r = 0; r < nr; ++r) a.conn[idx * nr + r] = -1;
+      __hip_atomic_store(&a.sinks[idx], 0u, __ATOMIC_RELAXED, WG);
+      __hip_atomic_store(&a.table[slot[u]], (uint32_t)idx, __ATOMIC_RELAXED, WG);
+      ++idx;
+    }
+    __syncthreads();
+    for (int t = tid; t < added * nr; t += kSmallThreads)
+      row_connect<NS, WG>(a.table, a.mask, a.states, a.stoich, ns, nr, n + t / nr, t % nr, a.conn, a.sinks);
+    __syncthreads();
+    // the next level explores the states just added, in ascending order
+    list = nullptr;
+    base = n;
+    nE = added;
+    n += added;
+  }
+  if (tid == 0) {
+    a.out[0] = level;
+    a.out[1] = n;
+    a.out[2] = base;
+    a.out[3] = nE;
+    a.out[4] = list ? 1 : 0;
   }
 }
 
@@ -214,6 +396,25 @@ __global__ void k_lookup(const uint32_t* table, uint64_t mask, const int32_t* st
 
 constexpr int kBlock = 256;
 
+// f with the kernels' species count as a constant: the next of 1, 2, 3, 4, 6, 8, 16
+template <class F>
+void by_species(int ns, F&& f) {
+  if (ns <= 1)
+    f(std::integral_constant<int, 1>{});
+  else if (ns == 2)
+    f(std::integral_constant<int, 2>{});
+  else if (ns == 3)
+    f(std::integral_constant<int, 3>{});
+  else if (ns == 4)
+    f(std::integral_constant<int, 4>{});
+  else if (ns <= 6)
+    f(std::integral_constant<int, 6>{});
+  else if (ns <= 8)
+    f(std::integral_constant<int, 8>{});
+  else
+    f(std::integral_constant<int, kMaxSpecies>{});
+}
+
 }  // namespace
 
 void space_reserve(nc_space_s* sp, int64_t rows) {
@@ -254,8 +455,10 @@ void space_add_candidates(nc_space_s* sp, int64_t n_cand) {
   sp->flags.reserve(n_cand);
   sp->ranks.reserve(n_cand);
   const uint64_t mask = sp->table_cap - 1;
-  k_cand_insert<<<grid_for(n_cand, kBlock), kBlock, 0, s>>>(sp->table.p, mask, sp->states.p, sp->cands.p, sp->ns,
-                                                             n_cand, sp->slot_of.p);
+  by_species(sp->ns, [&](auto NS) {
+    k_cand_insert<NS.value><<<grid_for(n_cand, kBlock), kBlock, 0, s>>>(sp->table.p, mask, sp->states.p, sp->cands.p,
+                                                                        sp->ns, n_cand, sp->slot_of.p);
+  });
   k_first_flags<<<grid_for(n_cand, kBlock), kBlock, 0, s>>>(sp->table.p, sp->slot_of.p, n_cand, sp->flags.p);
   NC_CHECK_HIP(hipGetLastError());
   uint32_t added = 0;
@@ -268,9 +471,11 @@ void space_add_candidates(nc_space_s* sp, int64_t n_cand) {
   sp->n = n_old + added;
   if (added) {
     int64_t work = (int64_t)added * sp->nr;
-    k_connect_new<<<grid_for(work, kBlock), kBlock, 0, s>>>(sp->table.p, mask, sp->states.p, sp->d_stoich.p, sp->ns,
-                                                             sp->nr, n_old, sp->n, sp->state_conn.p,
-                                                             sp->sink_mask.p);
+    by_species(sp->ns, [&](auto NS) {
+      k_connect_new<NS.value><<<grid_for(work, kBlock), kBlock, 0, s>>>(sp->table.p, mask, sp->states.p, sp->d_stoich.p,
+                                                                        sp->ns, sp->nr, n_old, sp->n,
+                                                                        sp->state_conn.p, sp->sink_mask.p);
+    });
     NC_CHECK_HIP(hipGetLastError());
     sp->version++;
   }
@@ -288,11 +493,16 @@ static void space_expand(nc_space_s* sp, int levels, const std::vector<int32_t>&
     rmask |= 1u << rlist[k];
   }
   // first-level explorables: ascending indices with a sink on some listed reaction (:165-173)
-  int64_t nE = 0;
-  if (sp->n) {
+  int64_t nE = 0, base = 0;
+  const int32_t* E = nullptr;
+  int level = 0;
+  if (sp->n == 0 || rl.n == 0) return;
+  sp->explorables.reserve(std::max<int64_t>(sp->n, kSmallCands));
+  E = sp->explorables.p;
+  bool listed = sp->n > kSmallCands;  // a small space's explorables are found by the small levels
+  if (listed) {
     sp->flags.reserve(sp->n);
     sp->ranks.reserve(sp->n);
-    sp->explorables.reserve(sp->n);
     k_flag_explorable<<<grid_for(sp->n, kBlock), kBlock, 0, s>>>(sp->sink_mask.p, sp->n, rmask, select,
                                                                    sp->flags.p);
     uint32_t cnt = 0;
@@ -301,11 +511,48 @@ static void space_expand(nc_space_s* sp, int levels, const std::vector<int32_t>&
     NC_CHECK_HIP(hipGetLastError());
     nE = cnt;
   }
-  const int32_t* E = sp->explorables.p;
-  int64_t base = 0;
-  for (int level = 0; level < levels; ++level) {  // :176-192
-    int64_t n_cand = nE * rl.n;
-    if (n_cand == 0) break;
+  while (level < levels) {  // :176-192
+    if (!listed || (nE > 0 && nE * rl.n <= kSmallCands && sp->n <= kSmallStates)) {
+      // room for several such levels, so that the kernel rarely stops for want of it
+      const int64_t room = sp->n + (int64_t)kSmallCands * std::min(levels - level, 8);
+      space_reserve(sp, room);
+      if ((uint64_t)(2 * room) > sp->table_cap) space_rebuild_table(sp, room);
+      ExpandArgs a{};
+      a.table = sp->table.p;
+      a.mask = sp->table_cap - 1;
+      a.states = sp->states.p;
+      a.conn = sp->state_conn.p;
+      a.sinks = sp->sink_mask.p;
+      a.stoich = sp->d_stoich.p;
+      a.list = E ? sp->explorables.p : nullptr;
+      a.select = select;
+      a.ns = sp->ns;
+      a.nr = sp->nr;
+      a.levels = levels - level;
+      a.rmask = rmask;
+      a.n_flag = listed ? -1 : (int32_t)sp->n;
+      a.n = sp->n;
+      a.nE = nE;
+      a.base = base;
+      a.max_rows = std::min<int64_t>(sp->cap, (int64_t)(sp->table_cap / 2));
+      a.rl = rl;
+      int64_t* out = static_cast<int64_t*>(host_stage(6));
+      NC_CHECK_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&a.out), out, 0));
+      by_species(sp->ns, [&](auto NS) { k_expand_small<NS.value><<<1, kSmallThreads, 0, s>>>(a); });
+      NC_CHECK_HIP(hipGetLastError());
+      NC_CHECK_HIP(hipStreamSynchronize(s));
+      level += (int)out[0];
+      if (out[1] > sp->n) sp->version++;
+      sp->n = out[1];
+      base = out[2];
+      nE = out[3];
+      if (!out[4]) E = nullptr;
+      listed = true;
+      if (nE == 0) break;
+      if (out[0] > 0) continue;  // stopped for rows (or done): the next round makes room
+    }
+    const int64_t n_cand = nE * rl.n;
+    if (n_cand == 0 || level >= levels) break;
     NC_REQUIRE(n_cand < (int64_t)0x7FFFFFF0, NC_ERR_OVERFLOW, "too many expansion candidates");
     sp->cands.reserve((size_t)n_cand * sp->ns);
     k_gen_candidates<<<grid_for(n_cand, kBlock), kBlock, 0, s>>>(sp->states.p, sp->d_stoich.p, sp->ns, E, base, nE,
@@ -317,6 +564,7 @@ static void space_expand(nc_space_s* sp, int levels, const std::vector<int32_t>&
     E = nullptr;
     base = n_old;
     nE = sp->n - n_old;
+    ++level;
   }
 }
 
