@@ -348,19 +348,36 @@ __global__ __launch_bounds__(kThreads) void k_mlp_train(const float* __restrict_
   if (tid == 0) loss_part[blockIdx.x] = ((r0[kNP] + r0[kRed + kNP]) + r0[2 * kRed + kNP]) + r0[3 * kRed + kNP];
 }
 
-// grad[p] = sum_b part[b][p] / count (fixed order); loss likewise
-__global__ void k_mlp_fold(int nblocks, const float* part, const float* loss_part, float inv_count, float* grad,
-                           float* loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kNP) {
-    float g = 0.0f;
-    for (int b = 0; b < nblocks; ++b) g += part[(int64_t)b * kNP + p];
-    grad[p] = g * inv_count;
+// grad[p] = sum_b part[b][p] / count, loss likewise, in a fixed order: wave w of a workgroup
+// adds partials w, w + 8, ... of 64 parameters, sixteen loads in flight, and the wave sums
+// are added in order. One thread per parameter waited for each of up to 512 loads in turn:
+// 143 us a gradient, 7 now.
+constexpr int kFoldWaves = 8;
+__global__ __launch_bounds__(64 * kFoldWaves) void k_mlp_fold(int nblocks, const float* part, const float* loss_part,
+                                                              float inv_count, float* grad, float* loss) {
+  constexpr int U = 16;
+  __shared__ float s_sum[kFoldWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane;  // kNP: the loss
+  const float* src = p < kNP ? part + p : loss_part;
+  const int64_t stride = p < kNP ? kNP : 1;
+  float acc = 0.0f;
+  for (int b = wave; b < nblocks; b += U * kFoldWaves) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = src[(int64_t)min(b + u * kFoldWaves, nblocks - 1) * stride];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc += b + u * kFoldWaves < nblocks ? v[u] : 0.0f;
   }
-  if (p == 0) {
-    float l = 0.0f;
-    for (int b = 0; b < nblocks; ++b) l += loss_part[b];
-    *loss = l * inv_count;
+  s_sum[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0) {
+    float t = s_sum[0][lane];
+#pragma unroll
+    for (int w = 1; w < kFoldWaves; ++w) t += s_sum[w][lane];
+    if (p < kNP) grad[p] = t * inv_count;
+    if (p == kNP) *loss = t * inv_count;
   }
 }
 
@@ -398,7 +415,7 @@ double mlp_grad_device(nc_mlp_s* M, int64_t n, const float* d_x, const float* d_
   M->part.reserve((size_t)std::max(nb, 1) * kNP);
   M->loss_part.reserve(std::max(nb, 1));
   k_mlp_train<<<nb, kThreads, 0, s>>>(d_x, d_y, n, M->params.p, M->part.p, M->loss_part.p);
-  k_mlp_fold<<<grid_for(kNP, 256), 256, 0, s>>>(nb, M->part.p, M->loss_part.p, 1.0f / (float)n, M->grad.p,
+  k_mlp_fold<<<grid_for(kNP + 1, 64), 64 * kFoldWaves, 0, s>>>(nb, M->part.p, M->loss_part.p, 1.0f / (float)n, M->grad.p,
                                                M->loss.p);
   NC_CHECK_HIP(hipGetLastError());
   float l = 0.0f;
@@ -518,7 +535,7 @@ int nc_mlp_train(nc_mlp M, int64_t n, const float* x, const float* y, int32_t ep
         M->part.reserve((size_t)blocks * kNP);
         M->loss_part.reserve(blocks);
         k_mlp_train<<<blocks, kThreads, 0, s>>>(bx.p, by.p, nb, M->params.p, M->part.p, M->loss_part.p);
-        k_mlp_fold<<<grid_for(kNP, 256), 256, 0, s>>>(blocks, M->part.p, M->loss_part.p, 1.0f / (float)nb, M->grad.p,
+        k_mlp_fold<<<grid_for(kNP + 1, 64), 64 * kFoldWaves, 0, s>>>(blocks, M->part.p, M->loss_part.p, 1.0f / (float)nb, M->grad.p,
                                                      M->loss.p);
         ++M->step;
         const float c1 = 1.0f - std::pow(b1, (float)M->step), c2 = 1.0f - std::pow(b2, (float)M->step);
