@@ -750,7 +750,7 @@ __device__ inline void err_sink(const MatArgs<VT>& a, int64_t blocks, int q, dou
 
 // Rows [i0, i0 + R) of the stored generator: out = A v (plus out when accumulating), the
 // FP64 row sums left in acc and v at the rows in vi (0 past the states).
-template <typename VT, typename OT, int KT, int R, int DM>
+template <typename VT, typename OT, int KT, int R, int DM, bool TV = false>
 __device__ __forceinline__ void stored_rows(const MatArgs<VT>& a, const VT* __restrict__ v, OT* __restrict__ out,
                                             int64_t i0, int accumulate, double (&acc)[R], double (&vi)[R]) {
   // Loads are unconditional (clamped indices, selects) and issued in two batches: the
@@ -783,6 +783,11 @@ __device__ __forceinline__ void stored_rows(const MatArgs<VT>& a, const VT* __re
     }
     return c;
   };
+  // TV: the first time-varying slot's loads go out with the others (a loop over the slots
+  // waits for each)
+  Pack<VT, R> td, tw;
+  Pack<int32_t, R> tc;
+  double tg[R];
   if constexpr (KT > 0) {
     // values and columns (computed columns need no load), then every gather; with
     // computed columns the gathers go out with the values, one round trip in all
@@ -793,11 +798,20 @@ __device__ __forceinline__ void stored_rows(const MatArgs<VT>& a, const VT* __re
       w[k] = ldpack<VT, R>(a.val + k * a.ld + i0);
       c[k] = slot_cols(k);
     }
+    if constexpr (TV) {
+      td = ldpack<VT, R>(a.tvd + i0);
+      tw = ldpack<VT, R>(a.tvv + i0);
+      tc = ldpack<int32_t, R>(a.tvc + i0);
+    }
     double gv[KT][R];
 #pragma unroll
     for (int k = 0; k < KT; ++k) {
 #pragma unroll
       for (int r = 0; r < R; ++r) gv[k][r] = (double)v[c[k].v[r]];
+    }
+    if constexpr (TV) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) tg[r] = (double)v[tc.v[r]];
     }
     __builtin_amdgcn_sched_barrier(0);
     // diag * v_i, then one fused multiply-add per slot in slot order (written out, so
@@ -819,7 +833,12 @@ __device__ __forceinline__ void stored_rows(const MatArgs<VT>& a, const VT* __re
       for (int r = 0; r < R; ++r) acc[r] = __fma_rn((double)w.v[r], (double)v[c.v[r]], acc[r]);
     }
   }
-  for (int q = 0; q < a.ntv; ++q) {
+  if constexpr (TV) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      acc[r] += a.tv_scale[0] * ((double)td.v[r] * vi[r] + (double)tw.v[r] * tg[r]);
+  }
+  for (int q = TV ? 1 : 0; q < a.ntv; ++q) {
     const Pack<VT, R> d = ldpack<VT, R>(a.tvd + q * a.ld + i0);
     const Pack<int32_t, R> c = ldpack<int32_t, R>(a.tvc + q * a.ld + i0);
     const Pack<VT, R> w = ldpack<VT, R>(a.tvv + q * a.ld + i0);
@@ -839,7 +858,7 @@ __device__ __forceinline__ void stored_rows(const MatArgs<VT>& a, const VT* __re
 // the next DP5(4) stage input (rk_epilogue) for its rows, state and sink rows alike.
 // ERR: the launch also forms the DP5(4) error sums of its rows (err_row), one per row
 // workgroup and one per sink row, and the sink values of the event check.
-template <typename VT, typename OT, int KT, int R, int DM, bool EPI = false, bool ERR = false>
+template <typename VT, typename OT, int KT, int R, int DM, bool EPI = false, bool ERR = false, bool TV = false>
 __global__ __launch_bounds__(kBlock) void k_matvec(MatArgs<VT> a, const VT* __restrict__ v, OT* __restrict__ out,
                                                    int accumulate) {
   const int64_t row_threads = (a.n + R - 1) / R;
@@ -856,7 +875,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec(MatArgs<VT> a, const VT* __re
       double r2 = 0.0;
       if (i0 < a.n) {
         double vi[R], acc[R];
-        stored_rows<VT, OT, KT, R, DM>(a, v, out, i0, accumulate, acc, vi);
+        stored_rows<VT, OT, KT, R, DM, TV>(a, v, out, i0, accumulate, acc, vi);
 #pragma unroll
         for (int r = 0; r < R; ++r)
           if (i0 + r < a.n) r2 += err_row(a, i0 + r, acc[r]);
@@ -881,7 +900,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec(MatArgs<VT> a, const VT* __re
       return;
     }
     double vi[R], acc[R];
-    stored_rows<VT, OT, KT, R, DM>(a, v, out, i0, accumulate, acc, vi);
+    stored_rows<VT, OT, KT, R, DM, TV>(a, v, out, i0, accumulate, acc, vi);
     if constexpr (EPI) rk_epilogue<VT, R>(a, i0, a.n, acc);
   } else {
     const int c = (int)((int64_t)blockIdx.x - row_blocks);
@@ -969,57 +988,73 @@ struct LaunchCfg {
   hipEvent_t e0, e1;
 };
 
-template <typename VT, typename OT, int K, int R, int DM, bool EPI = false, bool ERR = false>
+template <typename VT, typename OT, int K, int R, int DM, bool EPI = false, bool ERR = false, bool TV = false>
 void launch_one(const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, OT* oo, int acc) {
   if (c.e0)
-    hipExtLaunchKernelGGL(k_matvec<VT, OT, K, R, DM, EPI, ERR>, dim3(c.grid), dim3(kBlock), 0, c.s, c.e0, c.e1, 0, a,
+    hipExtLaunchKernelGGL(k_matvec<VT, OT, K, R, DM, EPI, ERR, TV>, dim3(c.grid), dim3(kBlock), 0, c.s, c.e0, c.e1, 0, a,
                           vv, oo, acc);
   else
-    k_matvec<VT, OT, K, R, DM, EPI, ERR><<<c.grid, kBlock, 0, c.s>>>(a, vv, oo, acc);
+    k_matvec<VT, OT, K, R, DM, EPI, ERR, TV><<<c.grid, kBlock, 0, c.s>>>(a, vv, oo, acc);
+}
+
+// Column mode of up to 8 slots: computed (DM 1) when every slot's columns are, else loaded
+// (DM 0), the stored columns being there for every slot. (The generic kernel, which decides
+// slot by slot and waits for each, and the time-varying slot's loads behind the others took
+// a solve of the four-state gene on 37,636 states from 14.5 to 16.7 ms.) More slots take
+// the generic kernel (DM 2).
+inline bool all_computed(uint32_t mask, int K) {
+  const uint32_t all = K >= 32 ? 0xffffffffu : ((1u << K) - 1u);
+  return mask != 0u && (mask & all) == all;
 }
 
 // The error-epilogue kernels: FP64 output, 2 rows per thread, stored generator
-template <typename VT, int DM>
+template <typename VT, int DM, bool TV>
 void dispatch_err_kd(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, double* oo) {
   switch (K) {
-    case 1: launch_one<VT, double, 1, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 2: launch_one<VT, double, 2, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 3: launch_one<VT, double, 3, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 4: launch_one<VT, double, 4, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 5: launch_one<VT, double, 5, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 6: launch_one<VT, double, 6, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 7: launch_one<VT, double, 7, 2, DM, false, true>(c, a, vv, oo, 0); break;
-    case 8: launch_one<VT, double, 8, 2, DM, false, true>(c, a, vv, oo, 0); break;
+    case 1: launch_one<VT, double, 1, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 2: launch_one<VT, double, 2, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 3: launch_one<VT, double, 3, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 4: launch_one<VT, double, 4, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 5: launch_one<VT, double, 5, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 6: launch_one<VT, double, 6, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 7: launch_one<VT, double, 7, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
+    case 8: launch_one<VT, double, 8, 2, DM, false, true, TV>(c, a, vv, oo, 0); break;
     default: launch_one<VT, double, 0, 2, 2, false, true>(c, a, vv, oo, 0); break;
   }
 }
 
-// The epilogue kernels: FP64 output, 2 rows per thread, stored generator (loaded, computed
-// or mixed columns)
-template <typename VT, int DM>
+template <typename VT>
+void dispatch_err(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, double* oo) {
+  const bool tv = a.ntv > 0;
+  if (all_computed(a.dia_mask, K))
+    tv ? dispatch_err_kd<VT, 1, true>(K, c, a, vv, oo) : dispatch_err_kd<VT, 1, false>(K, c, a, vv, oo);
+  else
+    tv ? dispatch_err_kd<VT, 0, true>(K, c, a, vv, oo) : dispatch_err_kd<VT, 0, false>(K, c, a, vv, oo);
+}
+
+// The stage-epilogue kernels, likewise
+template <typename VT, int DM, bool TV>
 void dispatch_epi_kd(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, double* oo) {
   switch (K) {
-    case 1: launch_one<VT, double, 1, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 2: launch_one<VT, double, 2, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 3: launch_one<VT, double, 3, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 4: launch_one<VT, double, 4, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 5: launch_one<VT, double, 5, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 6: launch_one<VT, double, 6, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 7: launch_one<VT, double, 7, 2, DM, true>(c, a, vv, oo, 0); break;
-    case 8: launch_one<VT, double, 8, 2, DM, true>(c, a, vv, oo, 0); break;
-    default: launch_one<VT, double, 0, 2, 2, true>(c, a, vv, oo, 0); break;
+    case 1: launch_one<VT, double, 1, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 2: launch_one<VT, double, 2, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 3: launch_one<VT, double, 3, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 4: launch_one<VT, double, 4, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 5: launch_one<VT, double, 5, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 6: launch_one<VT, double, 6, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 7: launch_one<VT, double, 7, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    case 8: launch_one<VT, double, 8, 2, DM, true, false, TV>(c, a, vv, oo, 0); break;
+    default: launch_one<VT, double, 0, 2, 2, true, false>(c, a, vv, oo, 0); break;
   }
 }
 
 template <typename VT>
 void dispatch_epi(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, double* oo) {
-  const uint32_t all = K >= 32 ? 0xffffffffu : ((1u << K) - 1u);
-  if (a.dia_mask == 0u)
-    dispatch_epi_kd<VT, 0>(K, c, a, vv, oo);
-  else if ((a.dia_mask & all) == all)
-    dispatch_epi_kd<VT, 1>(K, c, a, vv, oo);
+  const bool tv = a.ntv > 0;
+  if (all_computed(a.dia_mask, K))
+    tv ? dispatch_epi_kd<VT, 1, true>(K, c, a, vv, oo) : dispatch_epi_kd<VT, 1, false>(K, c, a, vv, oo);
   else
-    launch_one<VT, double, 0, 2, 2, true>(c, a, vv, oo, 0);
+    tv ? dispatch_epi_kd<VT, 0, true>(K, c, a, vv, oo) : dispatch_epi_kd<VT, 0, false>(K, c, a, vv, oo);
 }
 
 template <typename VT, typename OT, int R, int DM>
@@ -1037,17 +1072,12 @@ void dispatch_kd(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, 
   }
 }
 
-// Column mode: every slot loaded (0) or computed (1) takes the fixed-K kernels; a mix of
-// the two takes the generic kernel, which decides per slot.
 template <typename VT, typename OT, int R>
 void dispatch_k(int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT* vv, OT* oo, int acc) {
-  const uint32_t all = K >= 32 ? 0xffffffffu : ((1u << K) - 1u);
-  if (a.dia_mask == 0u)
-    dispatch_kd<VT, OT, R, 0>(K, c, a, vv, oo, acc);
-  else if ((a.dia_mask & all) == all)
+  if (all_computed(a.dia_mask, K))
     dispatch_kd<VT, OT, R, 1>(K, c, a, vv, oo, acc);
   else
-    launch_one<VT, OT, 0, R, 2>(c, a, vv, oo, acc);
+    dispatch_kd<VT, OT, R, 0>(K, c, a, vv, oo, acc);
 }
 
 // Launches of the computed modes (FP64 output, 1 or 2 rows per thread; DM 3: computed
@@ -1168,13 +1198,7 @@ void launch_matvec_t(nc_matrix_s* A, double t, const void* v, void* out, bool ac
     a.err_part = err->part;
     a.err_ex = err->ex;
     a.err_nex = err->n_ex;
-    const uint32_t all = A->K >= 32 ? 0xffffffffu : ((1u << A->K) - 1u);
-    if (a.dia_mask == 0u)
-      dispatch_err_kd<VT, 0>(A->K, c, a, vv, reinterpret_cast<double*>(out));
-    else if ((a.dia_mask & all) == all)
-      dispatch_err_kd<VT, 1>(A->K, c, a, vv, reinterpret_cast<double*>(out));
-    else
-      launch_one<VT, double, 0, 2, 2, false, true>(c, a, vv, reinterpret_cast<double*>(out), 0);
+    dispatch_err<VT>(A->K, c, a, vv, reinterpret_cast<double*>(out));
     return;
   }
   if (out_fp64 && A->mf_mode)
@@ -1454,13 +1478,10 @@ void launch_krylov_t(nc_matrix_s* A, hipStream_t s, const IopArgs& p, hipEvent_t
   const bool stored = p.c == 0;
   const MatArgs<VT> a = mat_args<VT>(A, 0.0);
   const LaunchCfg c{(unsigned)(p.groups + A->nr), s, e0, e1};
-  const uint32_t all = A->K >= 32 ? 0xffffffffu : ((1u << A->K) - 1u);
-  if (a.dia_mask == 0u)
-    dispatch_col_kd<VT, 0>(stored, A->K, c, a, p);
-  else if ((a.dia_mask & all) == all)
+  if (all_computed(a.dia_mask, A->K))
     dispatch_col_kd<VT, 1>(stored, A->K, c, a, p);
   else
-    launch_col<VT, 0, 2>(stored, c, a, p);
+    dispatch_col_kd<VT, 0>(stored, A->K, c, a, p);
 }
 
 // ---- matrix-free setup --------------------------------------------------------------
@@ -1893,7 +1914,7 @@ double matrix_bytes_per_matvec(const nc_matrix_s* A) {
   const double n = (double)A->n;
   double b = n * 8.0                                  // diag
              + n * A->K * (4.0 + vs)                  // ELL slots
-             - n * __builtin_popcount(A->dia_mask) * 4.0  // computed columns
+             - (A->K > 8 || all_computed(A->dia_mask, A->K) ? n * __builtin_popcount(A->dia_mask) * 4.0 : 0.0)  // computed columns
              + n * A->tv_r.size() * (4.0 + 2.0 * vs)  // time-varying slots
              + (double)A->n_sink_entries * (4.0 + vs)  // sink lists
              + (double)(A->nr + 1) * 8.0;

@@ -481,10 +481,10 @@ void launch_sens(nc_sensmatrix_s* SA, double t, const void* v, int64_t vstride, 
   };
   static_assert(kMaxSensBlocks <= 8 * (kBlock / 64), "blocks per wave");
   if (epi) {
-    // the stage epilogue kernels (FP32 storage, at most 4 blocks per wave: P + 1 <= 16)
-    if (!sens_rk_fusable(SA) || !std::is_same<VT, float>::value)
+    // the stage epilogue kernels (at most 4 blocks per wave: P + 1 <= 16)
+    if (!sens_rk_fusable(SA))
       throw Error(NC_ERR_INTERNAL, "sensitivity mat-vec epilogue not available");
-    if constexpr (std::is_same<VT, float>::value) {
+    {
       for (int j = 0; j < 6; ++j) {
         const bool on = (epi->mask >> j) & 1;
         a.rk_k[j] = on ? epi->k[j] : epi->k[0];
@@ -551,9 +551,14 @@ void launch_sens(nc_sensmatrix_s* SA, double t, const void* v, int64_t vstride, 
 
 }  // namespace
 
-// FP32 storage only: with FP64 stage-input copies the epilogue kernel measured 3% slower
-// over the C3 solve than the separate stage passes (8% faster in FP32 storage)
-bool sens_rk_fusable(const nc_sensmatrix_s* SA) { return SA->P + 1 <= 16 && SA->A->precision == NC_FP32; }
+// With FP64 stage-input copies the epilogue kernel measured 3% slower over a solve of 13
+// blocks on 262,144 states than the separate stage passes (8% faster in FP32 storage); below
+// 2^18 rows in all blocks the passes are launch latency: 13 blocks on 9,216 states took 25.7 ms
+// with them and 20.1 with the epilogue
+bool sens_rk_fusable(const nc_sensmatrix_s* SA) {
+  return SA->P + 1 <= 16 &&
+         (SA->A->precision == NC_FP32 || (int64_t)(SA->P + 1) * SA->A->n_rows <= (int64_t(1) << 18));
+}
 
 void sens_matvec_launch(nc_sensmatrix_s* SA, double t, const void* v, int64_t vstride, double* out, int64_t ostride,
                         hipStream_t s, const RkEpilogue* epi) {
