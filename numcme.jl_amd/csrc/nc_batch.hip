@@ -49,14 +49,17 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-__constant__ double c_a[7][6] = {
-    {0, 0, 0, 0, 0, 0},
-    {1.0 / 5, 0, 0, 0, 0, 0},
-    {3.0 / 40, 9.0 / 40, 0, 0, 0, 0},
-    {44.0 / 45, -56.0 / 15, 32.0 / 9, 0, 0, 0},
-    {19372.0 / 6561, -25360.0 / 2187, 64448.0 / 6561, -212.0 / 729, 0, 0},
-    {9017.0 / 3168, -355.0 / 33, 46732.0 / 5247, 49.0 / 176, -5103.0 / 18656, 0},
-    {35.0 / 384, 0, 500.0 / 1113, 125.0 / 192, -2187.0 / 6784, 11.0 / 84}};
+#define NC_BATCH_DP_A { \
+    {0, 0, 0, 0, 0, 0}, \
+    {1.0 / 5, 0, 0, 0, 0, 0}, \
+    {3.0 / 40, 9.0 / 40, 0, 0, 0, 0}, \
+    {44.0 / 45, -56.0 / 15, 32.0 / 9, 0, 0, 0}, \
+    {19372.0 / 6561, -25360.0 / 2187, 64448.0 / 6561, -212.0 / 729, 0, 0}, \
+    {9017.0 / 3168, -355.0 / 33, 46732.0 / 5247, 49.0 / 176, -5103.0 / 18656, 0}, \
+    {35.0 / 384, 0, 500.0 / 1113, 125.0 / 192, -2187.0 / 6784, 11.0 / 84}}
+__constant__ double c_a[7][6] = NC_BATCH_DP_A;
+const double h_a[7][6] = NC_BATCH_DP_A;  // the same table for the host
+#undef NC_BATCH_DP_A
 __constant__ double c_e[7] = {71.0 / 57600, 0, -71.0 / 16695, 71.0 / 1920, -17253.0 / 339200, 22.0 / 525, -1.0 / 40};
 
 // Solve settings read by the captured kernels from device memory, so that one captured
@@ -113,12 +116,12 @@ __global__ __launch_bounds__(kBlock) void k_bstage(Dev d, int64_t ld, const doub
     for (int j = 0; j < STAGE; ++j) {
       if (STAGE == 6 && j == 1) continue;
 #pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] += c_a[STAGE][j] * kj[j].v[r];
+      for (int r = 0; r < R; ++r) acc[r] = __fma_rn(c_a[STAGE][j], kj[j].v[r], acc[r]);
     }
     Pack<VT, R> o;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      y.v[r] += h * acc[r];
+      y.v[r] = __fma_rn(h, acc[r], y.v[r]);
       o.v[r] = (VT)y.v[r];
     }
     if constexpr (STAGE == 6) *reinterpret_cast<Pack<double, R>*>(ytmp + n0) = y;
@@ -144,11 +147,79 @@ struct SinkSegs {
 // clamped to the instance's states (rows whose value is 0 may point anywhere), instead of
 // loading them; the other instances load theirs. A wave's rows lie in one granule, so the
 // instance, its kind and its offsets are uniform and the choice is a scalar branch.
-template <typename VT, int R, int KT, int DM>
+//
+// KIND 1: the launch that forms stage s also forms stage s + 1's input for its rows (state
+// rows here, sink rows in their segments; the mat-vec's input and the next one's are two
+// buffers), KIND 2: the last one also sums the error norm of its rows, per granule and per
+// sink segment. Each takes a pass's launch and a re-read of the new stage with it: an
+// iteration of 48 instances in 800 granules went from 64 us (six mat-vecs of 4.6, five
+// stage passes of 3.3, an error pass of 3.6, a fold of 2.9, the controller 9.2, accept 4.4)
+// to 51 (mat-vecs of 5.9 and 6.2, the controller with the fold 10.7, accept 4.8).
+template <typename VT>
+struct BEpi {
+  const double* k[6];  // stages 0 .. 5 (a stage not read: stage 0 again)
+  double a[7];         // KIND 1: the next stage's weights of k[j], a[6] the new stage's
+  int32_t mask;        // KIND 1: bit j: k[j] is read
+  const double* u;
+  double* ytmp;        // y_{n+1}: KIND 1 writes it where set, KIND 2 reads it
+  VT* vin;
+  const Params* par;
+  double* partials;    // KIND 2: per granule, then per sink segment
+  int64_t grans;
+};
+
+template <typename VT, int R>
+__device__ inline void bstage_rows(const BEpi<VT>& e, double h, int64_t n0, int64_t nend, const double (&kn)[R]) {
+  Pack<double, R> kj[6];
+#pragma unroll
+  for (int j = 0; j < 6; ++j) kj[j] = *reinterpret_cast<const Pack<double, R>*>(e.k[j] + n0);
+  Pack<double, R> y = *reinterpret_cast<const Pack<double, R>*>(e.u + n0);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    double acc = 0.0;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const double t = __fma_rn(e.a[j], kj[j].v[r], acc);
+      acc = ((e.mask >> j) & 1) ? t : acc;
+    }
+    acc = __fma_rn(e.a[6], kn[r], acc);
+    y.v[r] = __fma_rn(h, acc, y.v[r]);
+    if (n0 + r < nend) {
+      e.vin[n0 + r] = (VT)y.v[r];
+      if (e.ytmp) e.ytmp[n0 + r] = y.v[r];
+    }
+  }
+}
+
+template <typename VT, int R>
+__device__ inline double berr_rows(const BEpi<VT>& e, double h, int64_t n0, int64_t nend, const double (&k6)[R]) {
+  const double atol = e.par->atol, rtol = e.par->rtol;
+  Pack<double, R> kj[6];
+#pragma unroll
+  for (int j = 0; j < 6; ++j)
+    if (j != 1) kj[j] = *reinterpret_cast<const Pack<double, R>*>(e.k[j] + n0);  // e_1 = 0
+  const Pack<double, R> uu = *reinterpret_cast<const Pack<double, R>*>(e.u + n0);
+  const Pack<double, R> yy = *reinterpret_cast<const Pack<double, R>*>(e.ytmp + n0);
+  double sum = 0.0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    double x = 0.0;
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      if (j != 1) x = __fma_rn(c_e[j], kj[j].v[r], x);
+    x = __fma_rn(c_e[6], k6[r], x);
+    const double q = h * x / (atol + rtol * fmax(fabs(uu.v[r]), fabs(yy.v[r])));
+    if (n0 + r < nend) sum += q * q;
+  }
+  return sum;
+}
+
+template <typename VT, int R, int KT, int DM, int KIND>
 __global__ __launch_bounds__(kBlock) void k_bmatvec(Dev d, int64_t ld, int K, const double* diag, const int32_t* col,
                                                     const VT* val, const VT* v, double* out, SinkSegs sg,
                                                     const VT* sval, const int32_t* dia_off, const int32_t* dia_inst,
-                                                    int Kb) {
+                                                    int Kb, BEpi<VT> epi) {
+  static_assert(KIND == 0 || R * 64 == kGran, "a granule is one wave's rows in the fused forms");
   if ((int)blockIdx.x < sg.nseg) {
     // sink row of one (instance, reaction) segment: one workgroup, deterministic tree
     const int seg = blockIdx.x;
@@ -160,7 +231,14 @@ __global__ __launch_bounds__(kBlock) void k_bmatvec(Dev d, int64_t ld, int K, co
     acc = wave_sum(acc);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) out[sg.row[seg]] = part[0] + part[1] + part[2] + part[3];
+    if (threadIdx.x == 0) {
+      const int64_t o = sg.row[seg];
+      const double kn[1] = {part[0] + part[1] + part[2] + part[3]};
+      out[o] = kn[0];
+      const double h = d.h[sg.inst[seg]];
+      if constexpr (KIND == 1) bstage_rows<VT, 1>(epi, h, o, o + 1, kn);
+      if constexpr (KIND == 2) epi.partials[epi.grans + seg] = berr_rows<VT, 1>(epi, h, o, o + 1, kn);
+    }
     return;
   }
   const uint32_t nl = *d.n_agran;
@@ -169,60 +247,70 @@ __global__ __launch_bounds__(kBlock) void k_bmatvec(Dev d, int64_t ld, int K, co
     int64_t n0;
     if (!unit_rows<R>(d, nl, un, n0)) continue;
     const int inst = __builtin_amdgcn_readfirstlane(d.gran_inst[n0 / kGran]);
-    if (d.h[inst] == 0.0) continue;
+    const double h = d.h[inst];
+    if (h == 0.0) continue;
     const int64_t nbeg = d.row_off[inst], nend = nbeg + d.nstates[inst];
-    if (n0 >= nend) continue;
-    const Pack<double, R> dg = *reinterpret_cast<const Pack<double, R>*>(diag + n0);
-    const Pack<VT, R> vi = *reinterpret_cast<const Pack<VT, R>*>(v + n0);
-    double acc[R];
-    if constexpr (KT > 0) {
-      Pack<int32_t, R> c[KT];
-      Pack<VT, R> w[KT];
-      if (DM == 1 && dia_inst[inst]) {
+    if (KIND != 2 && n0 >= nend) continue;
+    double err = 0.0;
+    if (n0 < nend) {
+      const Pack<double, R> dg = *reinterpret_cast<const Pack<double, R>*>(diag + n0);
+      const Pack<VT, R> vi = *reinterpret_cast<const Pack<VT, R>*>(v + n0);
+      double acc[R];
+      if constexpr (KT > 0) {
+        Pack<int32_t, R> c[KT];
+        Pack<VT, R> w[KT];
+        if (DM == 1 && dia_inst[inst]) {
+#pragma unroll
+          for (int s = 0; s < KT; ++s) {
+            const int64_t off = dia_off[(int64_t)inst * Kb + s];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const int64_t j = n0 + r + off;
+              c[s].v[r] = (int32_t)(j < nbeg ? nbeg : (j >= nend ? nend - 1 : j));
+            }
+            w[s] = *reinterpret_cast<const Pack<VT, R>*>(val + (int64_t)s * ld + n0);
+          }
+        } else {
+#pragma unroll
+          for (int s = 0; s < KT; ++s) {
+            c[s] = *reinterpret_cast<const Pack<int32_t, R>*>(col + (int64_t)s * ld + n0);
+            w[s] = *reinterpret_cast<const Pack<VT, R>*>(val + (int64_t)s * ld + n0);
+          }
+        }
+        double gv[KT][R];
 #pragma unroll
         for (int s = 0; s < KT; ++s) {
-          const int64_t off = dia_off[(int64_t)inst * Kb + s];
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const int64_t j = n0 + r + off;
-            c[s].v[r] = (int32_t)(j < nbeg ? nbeg : (j >= nend ? nend - 1 : j));
-          }
-          w[s] = *reinterpret_cast<const Pack<VT, R>*>(val + (int64_t)s * ld + n0);
+          for (int r = 0; r < R; ++r) gv[s][r] = (double)v[c[s].v[r]];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r] = dg.v[r] * (double)vi.v[r];
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[r] += (double)w[s].v[r] * gv[s][r];
         }
       } else {
 #pragma unroll
-        for (int s = 0; s < KT; ++s) {
-          c[s] = *reinterpret_cast<const Pack<int32_t, R>*>(col + (int64_t)s * ld + n0);
-          w[s] = *reinterpret_cast<const Pack<VT, R>*>(val + (int64_t)s * ld + n0);
+        for (int r = 0; r < R; ++r) acc[r] = dg.v[r] * (double)vi.v[r];
+        for (int s = 0; s < K; ++s) {
+          const Pack<int32_t, R> c = *reinterpret_cast<const Pack<int32_t, R>*>(col + (int64_t)s * ld + n0);
+          const Pack<VT, R> w = *reinterpret_cast<const Pack<VT, R>*>(val + (int64_t)s * ld + n0);
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[r] += (double)w.v[r] * (double)v[c.v[r]];
         }
       }
-      double gv[KT][R];
 #pragma unroll
-      for (int s = 0; s < KT; ++s) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) gv[s][r] = (double)v[c[s].v[r]];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = dg.v[r] * (double)vi.v[r];
-#pragma unroll
-      for (int s = 0; s < KT; ++s) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += (double)w[s].v[r] * gv[s][r];
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = dg.v[r] * (double)vi.v[r];
-      for (int s = 0; s < K; ++s) {
-        const Pack<int32_t, R> c = *reinterpret_cast<const Pack<int32_t, R>*>(col + (int64_t)s * ld + n0);
-        const Pack<VT, R> w = *reinterpret_cast<const Pack<VT, R>*>(val + (int64_t)s * ld + n0);
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += (double)w.v[r] * (double)v[c.v[r]];
-      }
+      for (int r = 0; r < R; ++r)
+        if (n0 + r < nend) out[n0 + r] = acc[r];
+      if constexpr (KIND == 1) bstage_rows<VT, R>(epi, h, n0, nend, acc);
+      if constexpr (KIND == 2) err = berr_rows<VT, R>(epi, h, n0, nend, acc);
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (n0 + r < nend) out[n0 + r] = acc[r];
+    if constexpr (KIND == 2) {
+      err = wave_sum(err);
+      if ((threadIdx.x & 63) == 0) epi.partials[n0 / kGran] = err;
+    }
   }
 }
 
@@ -279,19 +367,26 @@ __global__ __launch_bounds__(kBlock) void k_berr(Dev d, int64_t ld, const Params
   }
 }
 
-// Per-instance fold of the granule partials (granules of an instance are contiguous): one
-// wavefront per instance, lane l adding granules l, l + 64, ... in order, then a fixed
-// shuffle tree (deterministic)
-__global__ __launch_bounds__(kBlock) void k_bfold(int n_inst, const int64_t* gran_start, const double* h,
-                                                  const double* partials, double* err) {
-  const int i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+// An instance's error sum: lane l of a wave adds granule partials l, l + 64, ... in order,
+// then (the fused error sums) its sink segments', then a fixed shuffle tree (deterministic).
+// Granules and segments of an instance are contiguous.
+__device__ inline double fold_instance(int i, const int64_t* gran_start, const int32_t* seg_start, int64_t grans,
+                                       const double* partials) {
   const int lane = threadIdx.x & 63;
-  if (i >= n_inst) return;  // whole wavefronts leave together
-  if (h[i] == 0.0) return;  // not stepped in this iteration: its partials are stale
   double sum = 0.0;
   for (int64_t g = gran_start[i] + lane; g < gran_start[i + 1]; g += 64) sum += partials[g];
-  sum = wave_sum(sum);
-  if (lane == 0) err[i] = sum;
+  if (seg_start)
+    for (int q = seg_start[i] + lane; q < seg_start[i + 1]; q += 64) sum += partials[grans + q];
+  return wave_sum(sum);
+}
+
+__global__ __launch_bounds__(kBlock) void k_bfold(int n_inst, const int64_t* gran_start, const int32_t* seg_start,
+                                                  int64_t grans, const double* h, const double* partials, double* err) {
+  const int i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (i >= n_inst) return;  // whole wavefronts leave together
+  if (h[i] == 0.0) return;  // not stepped in this iteration: its partials are stale
+  const double sum = fold_instance(i, gran_start, seg_start, grans, partials);
+  if ((threadIdx.x & 63) == 0) err[i] = sum;
 }
 
 // Accept the last step where asked (u <- y, k0 <- k6) and fill requested snapshots.
@@ -353,7 +448,10 @@ struct Ctl {
   int n;
   const Params* par;
   const double* t_out;
-  const double* err;        // folded error sums of the iteration just run
+  double* err;              // folded error sums of the iteration just run
+  const double* partials;   // not null: the controller folds them itself
+  const int32_t* seg_start;
+  int64_t grans;
   const int64_t* nrows;     // error norm length per instance
   const int64_t* gran_start;
   double* t;                // current time
@@ -373,7 +471,7 @@ struct Ctl {
   uint32_t* counters;       // [0] instances still running, [1] iterations with work
 };
 
-__device__ void control_one(const Ctl& c, int i, bool init, int n_out, double h0, int64_t max_steps) {
+__device__ void control_one(const Ctl& c, int i, bool init, int n_out, double h0, int64_t max_steps, double err_sum) {
   if (init) {
     c.t[i] = n_out ? c.t_out[0] : 0.0;
     c.next[i] = 1;
@@ -388,7 +486,7 @@ __device__ void control_one(const Ctl& c, int i, bool init, int n_out, double h0
     c.hc[i] = h0 > 0 ? h0 : 1e-3 * fmax(1e-12, tend - c.t[i]);
   } else if (c.htry[i] != 0.0) {
     const double hs = c.htry[i];
-    const double err = sqrt(c.err[i] / (double)c.nrows[i]);
+    const double err = sqrt(err_sum / (double)c.nrows[i]);
     c.accept[i] = 0;
     c.snap[i] = -1;
     if (!isfinite(err)) {
@@ -464,16 +562,38 @@ __device__ uint32_t block_scan(uint32_t v, uint32_t* sh, uint32_t& total) {
 // with work in the next iteration (a step to take, or an accept / snapshot to apply).
 __global__ __launch_bounds__(kCtlBlock) void k_bcontrol(Ctl c, int init) {
   __shared__ uint32_t sh[kCtlBlock / 64 + 1];
-  __shared__ int any;
-  if (threadIdx.x == 0) any = 0;
+  __shared__ double s_err[kCtlBlock];
+  __shared__ int any, changed;
+  if (threadIdx.x == 0) any = 0, changed = init;
   __syncthreads();
   const int n_out = c.par->n_out;
   const double h0 = c.par->h0;
   const int64_t max_steps = c.par->max_steps;
+  // the error sums: sixteen lanes an instance, so that up to 64 instances' dependent loads
+  // (range, then partials) are in flight at once
+  if (!init && c.partials) {
+    const int lane = threadIdx.x & 15;
+    for (int i = threadIdx.x >> 4; i < c.n; i += kCtlBlock / 16) {
+      double sum = 0.0;
+      const int64_t g0 = c.gran_start[i], g1 = c.gran_start[i + 1];
+      const int q0 = c.seg_start ? c.seg_start[i] : 0, q1 = c.seg_start ? c.seg_start[i + 1] : 0;
+      for (int64_t g = g0 + lane; g < g1; g += 16) sum += c.partials[g];
+      for (int q = q0 + lane; q < q1; q += 16) sum += c.partials[c.grans + q];
+      for (int off = 8; off > 0; off >>= 1) sum += __shfl_down(sum, off, 16);
+      if (lane == 0) {
+        if (i < kCtlBlock)
+          s_err[i] = sum;
+        else
+          c.err[i] = sum;
+      }
+    }
+  }
+  __syncthreads();
   uint32_t running = 0;
   for (int i = threadIdx.x; i < c.n; i += kCtlBlock) {
     if (!init && c.htry[i] != 0.0) atomicOr(&any, 1);
-    control_one(c, i, init != 0, n_out, h0, max_steps);
+    control_one(c, i, init != 0, n_out, h0, max_steps,
+                init ? 0.0 : (c.partials && i < kCtlBlock ? s_err[i] : c.err[i]));
     running += c.htry[i] != 0.0;
   }
   // instance offsets into the list, in instance order
@@ -485,10 +605,16 @@ __global__ __launch_bounds__(kCtlBlock) void k_bcontrol(Ctl c, int init) {
       cnt = (uint32_t)(c.gran_start[i + 1] - c.gran_start[i]);
     uint32_t tot;
     const uint32_t o = block_scan(cnt, sh, tot);
-    if (i < c.n) c.off[i] = carry + o;
+    if (i < c.n && c.off[i] != carry + o) {
+      c.off[i] = carry + o;
+      changed = 1;
+    }
     carry += tot;
   }
-  if (threadIdx.x == 0) c.off[c.n] = carry;
+  if (threadIdx.x == 0 && c.off[c.n] != carry) {
+    c.off[c.n] = carry;
+    changed = 1;
+  }
   // running count: one wave sum per wave, then atomics (ordering-free: integers)
   __shared__ uint32_t nrun;
   if (threadIdx.x == 0) nrun = 0;
@@ -497,8 +623,9 @@ __global__ __launch_bounds__(kCtlBlock) void k_bcontrol(Ctl c, int init) {
   __syncthreads();
   // the list: instance i's granules at entries [off[i], off[i + 1]), written by one wave
   // per instance (instances dealt to the waves in turn), 64 consecutive entries at a time
-  const uint32_t total = c.off[c.n];
-  {
+  // (the offsets tell the list: while no instance joins or leaves, it stands)
+  const uint32_t total = carry;
+  if (changed) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int i = wave; i < c.n; i += kCtlBlock / 64) {
       const uint32_t o0 = c.off[i], o1 = c.off[i + 1];
@@ -580,12 +707,13 @@ struct nc_batch_s {
   int nseg = 0;
   nc::DevBuf<int32_t> seg_inst, sink_src;
   nc::DevBuf<int64_t> seg_row, seg_off;
+  nc::DevBuf<int32_t> seg_start;  // n + 1: first segment of each instance
   nc::DevBuf<unsigned char> sink_val;
   nc::DevBuf<int32_t> gran_inst;
   nc::DevBuf<int64_t> d_row_off, d_nstates, d_gran_start, d_nrows;
   // integrator state
   nc::DevBuf<double> u, ytmp, k, partials, err, snaps;
-  nc::DevBuf<unsigned char> vin;
+  nc::DevBuf<unsigned char> vin, vin2;  // two stage inputs: the fused forms read one and write the other
   // controller state (per instance) and the active granule list
   nc::DevBuf<double> c_t, c_hc, d_h, t_out;
   nc::DevBuf<int32_t> c_next, c_done, c_clamped, d_accept, d_snap, c_status;
@@ -651,6 +779,10 @@ void batch_build(nc_batch_s* B, const nc_matrix_s* const* mats) {
       seg_off.push_back(total);
     }
   B->nseg = (int)seg_inst.size();
+  std::vector<int32_t> seg_start{0};
+  for (int i = 0; i < B->n; ++i) seg_start.push_back(seg_start.back() + mats[i]->nr);
+  B->seg_start.alloc(seg_start.size());
+  NC_CHECK_HIP(hipMemcpyAsync(B->seg_start.p, seg_start.data(), sizeof(int32_t) * seg_start.size(), hipMemcpyHostToDevice, s));
   B->seg_inst.alloc(std::max<size_t>(seg_inst.size(), 1));
   B->seg_row.alloc(std::max<size_t>(seg_row.size(), 1));
   B->seg_off.alloc(seg_off.size());
@@ -730,13 +862,15 @@ nc_batch_s* batch_create(int n, const nc_matrix* mats) {
   B->ytmp.alloc(ld);
   B->k.alloc((size_t)7 * ld);
   B->vin.alloc(ld * B->vs);
-  B->partials.alloc(B->grans);
+  B->vin2.alloc(ld * B->vs);
+  B->partials.alloc(B->grans + B->nseg);
   B->err.alloc(n);
   NC_CHECK_HIP(hipMemsetAsync(B->u.p, 0, sizeof(double) * ld, s));
   NC_CHECK_HIP(hipMemsetAsync(B->ytmp.p, 0, sizeof(double) * ld, s));
   NC_CHECK_HIP(hipMemsetAsync(B->k.p, 0, sizeof(double) * 7 * ld, s));
   NC_CHECK_HIP(hipMemsetAsync(B->vin.p, 0, B->vs * ld, s));
-  NC_CHECK_HIP(hipMemsetAsync(B->partials.p, 0, sizeof(double) * B->grans, s));
+  NC_CHECK_HIP(hipMemsetAsync(B->vin2.p, 0, B->vs * ld, s));
+  NC_CHECK_HIP(hipMemsetAsync(B->partials.p, 0, sizeof(double) * (B->grans + B->nseg), s));
   NC_CHECK_HIP(hipMemsetAsync(B->err.p, 0, sizeof(double) * n, s));
   B->c_t.alloc(n);
   B->c_hc.alloc(n);
@@ -769,6 +903,15 @@ Dev dev_view(nc_batch_s* B) {
              B->agran.p,     B->n_agran.p};
 }
 
+// The fused forms at the default launch shape, four rows per thread (a wave's rows are one
+// granule there); the other shapes run the stage and error passes.
+bool fused(const nc_batch_s* B) { return B->rows_per_thread == 4; }
+
+// Up to here the one-workgroup controller folds the error sums itself; more granules are
+// folded by a launch of their own first.
+constexpr int64_t kControllerGrans = 4096;
+bool controller_folds(const nc_batch_s* B) { return B->grans <= kControllerGrans; }
+
 Ctl ctl_view(nc_batch_s* B) {
   Ctl c{};
   c.n = B->n;
@@ -777,6 +920,9 @@ Ctl ctl_view(nc_batch_s* B) {
   c.err = B->err.p;
   c.nrows = B->d_nrows.p;
   c.gran_start = B->d_gran_start.p;
+  c.partials = controller_folds(B) ? B->partials.p : nullptr;
+  c.seg_start = fused(B) ? B->seg_start.p : nullptr;
+  c.grans = B->grans;
   c.t = B->c_t.p;
   c.hc = B->c_hc.p;
   c.htry = B->d_h.p;
@@ -800,28 +946,28 @@ unsigned row_grid(const nc_batch_s* B, int R) {
   return (unsigned)std::min<int64_t>((B->grans + R - 1) / R, kMaxRowBlocks);
 }
 
-template <typename VT, int R>
-void launch_matvec(nc_batch_s* B, const VT* v, double* out) {
+template <typename VT, int R, int KIND = 0>
+void launch_matvec(nc_batch_s* B, const VT* v, double* out, const BEpi<VT>& epi = BEpi<VT>{}) {
   const Dev d = dev_view(B);
   hipStream_t s = B->stream.s;
   const SinkSegs sg{(int32_t)B->nseg, B->seg_inst.p, B->seg_row.p, B->seg_off.p, B->sink_src.p};
   const unsigned grid = row_grid(B, R) + (unsigned)B->nseg;
   auto go = [&](auto kern) {
     kern<<<grid, kBlock, 0, s>>>(d, B->ld, B->K, B->diag.p, B->col.p, reinterpret_cast<const VT*>(B->val.p), v, out,
-                                 sg, reinterpret_cast<const VT*>(B->sink_val.p), B->dia_off.p, B->dia_inst.p, B->K);
+                                 sg, reinterpret_cast<const VT*>(B->sink_val.p), B->dia_off.p, B->dia_inst.p, B->K, epi);
   };
   auto by_k = [&](auto dm) {
     constexpr int DM = decltype(dm)::value;
     switch (B->K) {
-      case 1: go(k_bmatvec<VT, R, 1, DM>); break;
-      case 2: go(k_bmatvec<VT, R, 2, DM>); break;
-      case 3: go(k_bmatvec<VT, R, 3, DM>); break;
-      case 4: go(k_bmatvec<VT, R, 4, DM>); break;
-      case 5: go(k_bmatvec<VT, R, 5, DM>); break;
-      case 6: go(k_bmatvec<VT, R, 6, DM>); break;
-      case 7: go(k_bmatvec<VT, R, 7, DM>); break;
-      case 8: go(k_bmatvec<VT, R, 8, DM>); break;
-      default: go(k_bmatvec<VT, R, 0, 0>); break;
+      case 1: go(k_bmatvec<VT, R, 1, DM, KIND>); break;
+      case 2: go(k_bmatvec<VT, R, 2, DM, KIND>); break;
+      case 3: go(k_bmatvec<VT, R, 3, DM, KIND>); break;
+      case 4: go(k_bmatvec<VT, R, 4, DM, KIND>); break;
+      case 5: go(k_bmatvec<VT, R, 5, DM, KIND>); break;
+      case 6: go(k_bmatvec<VT, R, 6, DM, KIND>); break;
+      case 7: go(k_bmatvec<VT, R, 7, DM, KIND>); break;
+      case 8: go(k_bmatvec<VT, R, 8, DM, KIND>); break;
+      default: go(k_bmatvec<VT, R, 0, 0, KIND>); break;
     }
   };
   if (B->any_dia)
@@ -863,13 +1009,41 @@ void iteration_r(nc_batch_s* B, bool control) {
   const unsigned g = row_grid(B, R);
   k_baccept_stage1<VT, R><<<g, kBlock, 0, s>>>(d, B->ld, B->u.p, B->ytmp.p, B->k.p, B->snaps.p,
                                                reinterpret_cast<VT*>(B->vin.p));
-  for (int st = 1; st < 7; ++st) {
-    if (st > 1) launch_stage<VT, R>(B, st, g);
-    launch_matvec<VT, R>(B, reinterpret_cast<const VT*>(B->vin.p), B->k.p + (int64_t)st * B->ld);
+  if constexpr (R == 4) {
+    BEpi<VT> e{};
+    for (int j = 0; j < 6; ++j) e.k[j] = B->k.p + (int64_t)j * B->ld;
+    e.u = B->u.p;
+    e.par = B->par.p;
+    e.partials = B->partials.p;
+    e.grans = B->grans;
+    VT *cur = reinterpret_cast<VT*>(B->vin.p), *nxt = reinterpret_cast<VT*>(B->vin2.p);
+    for (int st = 1; st < 6; ++st) {
+      BEpi<VT> f = e;
+      f.mask = 0;
+      for (int j = 0; j < 6; ++j) {
+        const bool on = j < st && !(st + 1 == 6 && j == 1);  // a_61 = 0
+        f.mask |= on ? 1 << j : 0;
+        f.a[j] = on ? h_a[st + 1][j] : 0.0;
+        if (!on) f.k[j] = e.k[0];
+      }
+      f.a[6] = h_a[st + 1][st];
+      f.ytmp = st + 1 == 6 ? B->ytmp.p : nullptr;
+      f.vin = nxt;
+      launch_matvec<VT, R, 1>(B, cur, B->k.p + (int64_t)st * B->ld, f);
+      std::swap(cur, nxt);
+    }
+    e.ytmp = B->ytmp.p;
+    launch_matvec<VT, R, 2>(B, cur, B->k.p + (int64_t)6 * B->ld, e);
+  } else {
+    for (int st = 1; st < 7; ++st) {
+      if (st > 1) launch_stage<VT, R>(B, st, g);
+      launch_matvec<VT, R>(B, reinterpret_cast<const VT*>(B->vin.p), B->k.p + (int64_t)st * B->ld);
+    }
+    k_berr<R><<<g, kBlock, 0, s>>>(d, B->ld, B->par.p, B->u.p, B->ytmp.p, B->k.p, B->partials.p);
   }
-  k_berr<R><<<g, kBlock, 0, s>>>(d, B->ld, B->par.p, B->u.p, B->ytmp.p, B->k.p, B->partials.p);
-  k_bfold<<<(unsigned)((B->n + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, s>>>(B->n, B->d_gran_start.p, B->d_h.p,
-                                                                                B->partials.p, B->err.p);
+  if (!control || !controller_folds(B))
+    k_bfold<<<(unsigned)((B->n + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, s>>>(
+        B->n, B->d_gran_start.p, R == 4 ? B->seg_start.p : nullptr, B->grans, B->d_h.p, B->partials.p, B->err.p);
   NC_CHECK_HIP(hipGetLastError());
   if (control) launch_control(B, 0);
 }
