@@ -586,16 +586,16 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
     }
     const double avnorm = hb[L.misc(MISC_AVN)];
     const int mxf = mb + k1;  // size of the exponentiated matrix
-    std::vector<double> Hm((size_t)mxf * mxf, 0.0), F(mxf);  // F: first column of exp(tau Hm)
+    std::vector<double> F(mxf);  // first column of exp(tau H), H tridiagonal
     auto exp_tau = [&](double tau, std::vector<double>& out) {
-      for (int i = 0; i < mxf; ++i)
-        for (int jj = 0; jj < mxf; ++jj) {
-          double v = 0.0;
-          if (i < mb + 1 && jj < mb && i <= jj + 1 && i < m + 1) v = hb[L.H(i, jj)];
-          if (k1 != 0 && i == m + 1 && jj == m) v = 1.0;
-          Hm[(size_t)i * mxf + jj] = tau * v;
-        }
-      expm_first_column(mxf, Hm.data(), out.data());
+      double lo[34], di[34], up[34];  // m <= 31
+      auto h = [&](int i, int j) { return i < m + 1 && i < mb + 1 && j < mb ? tau * hb[L.H(i, j)] : 0.0; };
+      for (int i = 0; i < mxf; ++i) {
+        lo[i] = i > 0 ? (k1 != 0 && i == m + 1 ? tau : h(i, i - 1)) : 0.0;
+        di[i] = h(i, i);
+        up[i] = i + 1 < mxf ? h(i, i + 1) : 0.0;
+      }
+      expm_first_column(mxf, lo, di, up, out.data());
     };
     double err_loc = btol, xm = 1.0 / m;
     for (int ireject = 0;; ++ireject) {

@@ -38,23 +38,28 @@ void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, DevBuf<uns
 // ---- dense matrix exponential (host, FP64) --------------------------------------------
 // Scaling and squaring with the [13/13] Pade approximant and the theta_13 threshold of
 // N. J. Higham, "The scaling and squaring method for the matrix exponential revisited",
-// SIAM J. Matrix Anal. Appl. 26(4), 2005. The Krylov integrator calls it at least once per
-// step on its (m+2)x(m+2) Hessenberg matrix, between a device synchronisation and the next
-// launch, so it is on the solve's critical path: matrices of at most kExpmMax rows are
-// padded to a multiple of 8 and multiplied with a row of the product held in vector
-// registers (AVX2 and FMA when the host has them, checked once; plain vectors otherwise).
-// The Krylov step needs only the first column, which saves the last squaring.
+// SIAM J. Matrix Anal. Appl. 26(4), 2005. Matrices of at most kExpmMax rows are padded to a
+// multiple of 8 and multiplied with a row of the product held in vector registers (AVX2 and
+// FMA when the host has them, checked once; plain vectors otherwise).
+//
+// A Krylov step needs the first column of its tridiagonal (m+2)x(m+2) matrix at least once,
+// between a device synchronisation and the next launch, and some fifty times where it
+// locates an event: nc_expm_tri.h's Taylor form while its work, which grows with the norm,
+// is below the dense form's (m = 30: 6 us at norm 48 and 22 at norm 256, against 27 and
+// 29); the dense form's first column, which saves the last squaring, above that.
 namespace {
 
 constexpr int kExpmMax = 64;
 namespace expm_avx2 {
 #pragma clang attribute push(__attribute__((target("avx2,fma"))), apply_to = function)
 #include "nc_expm_impl.h"
+#include "nc_expm_tri.h"
 #pragma clang attribute pop
 }  // namespace expm_avx2
 
 namespace expm_base {
 #include "nc_expm_impl.h"
+#include "nc_expm_tri.h"
 }  // namespace expm_base
 
 bool host_has_avx2() {
@@ -162,14 +167,19 @@ void expm_dense(int n, const double* a, double* out) {
     expm_small(n, a, out, false);
 }
 
-void expm_first_column(int n, const double* a, double* out) {
-  if (n > kExpmMax) {
-    std::vector<double> full((size_t)n * n);
-    expm_large(n, a, full.data());
-    for (int i = 0; i < n; ++i) out[i] = full[(size_t)i * n];
-    return;
+void expm_first_column(int n, const double* lo, const double* di, const double* up, double* out) {
+  NC_REQUIRE(n > 0 && n <= kExpmMax, NC_ERR_INTERNAL, "tridiagonal exponential: size out of range");
+  constexpr int max_parts = 32;  // a norm of 256
+  const bool done = host_has_avx2() ? expm_avx2::expm_tri(n, lo, di, up, max_parts, out)
+                                    : expm_base::expm_tri(n, lo, di, up, max_parts, out);
+  if (done) return;
+  std::vector<double> a((size_t)n * n, 0.0);
+  for (int i = 0; i < n; ++i) {
+    if (i > 0) a[(size_t)i * n + i - 1] = lo[i];
+    a[(size_t)i * n + i] = di[i];
+    if (i + 1 < n) a[(size_t)i * n + i + 1] = up[i];
   }
-  expm_small(n, a, out, true);
+  expm_small(n, a.data(), out, true);
 }
 
 }  // namespace nc

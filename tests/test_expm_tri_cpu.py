@@ -1,0 +1,130 @@
+"""The first column of exp(T) of a tridiagonal T (the Taylor form a Krylov step uses, host
+code compiled here by itself) against the same column in extended precision: birth-death
+sections with the two augmentation rows of a step, matrices far from normal, shifts of either
+sign, every remainder of the vector width, and the norm above which the form declines.
+"""
+import ctypes
+import math
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+CSRC = Path(__file__).resolve().parents[1] / "numcme.jl_amd" / "csrc"
+EPS = np.finfo(float).eps
+
+
+@pytest.fixture(scope="module")
+def tri(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("tri")
+    src = d / "tri.cpp"
+    src.write_text("#include <algorithm>\n#include <cmath>\n#include \"nc_expm_tri.h\"\n"
+                   "extern \"C\" int tri(int n, const double* l, const double* d, const double* u, int p, double* o) "
+                   "{ return expm_tri(n, l, d, u, p, o); }\n")
+    lib = d / "tri.so"
+    subprocess.run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", str(src), "-o", str(lib)], check=True)
+    fn = ctypes.CDLL(str(lib)).tri
+    P = ctypes.POINTER(ctypes.c_double)
+
+    def run(lo, di, up, parts=32):
+        out = np.full(len(di), np.nan)
+        args = [np.ascontiguousarray(v, dtype=np.float64) for v in (lo, di, up)]
+        ok = fn(len(di), *(v.ctypes.data_as(P) for v in args), parts, out.ctypes.data_as(P))
+        return bool(ok), out
+
+    return run
+
+
+def column(lo, di, up):
+    """exp(T) e1 and the error bound of the form: with s parts of norm p after the shift c,
+    a part's terms grow to at most e^p and are damped by e^{-c/s}; each of its products and
+    sums (at most 4 + 48) rounds to eps of that."""
+    L = np.longdouble
+    lo, di, up = (np.asarray(v, dtype=L) for v in (lo, di, up))
+    c = -(di.min() + di.max()) / 2
+    d = di + c
+    n = len(di)
+    cols = np.abs(d)
+    cols[1:] += np.abs(up[:-1])
+    cols[:-1] += np.abs(lo[1:])
+    norm = float(cols.max())
+    s = 1
+    while norm > 8.0 * s or norm - c > 4.0 * s:
+        s *= 2
+    fine = 4 * s
+    v = np.zeros(n, L)
+    v[0] = 1
+    big = L(1)
+    for _ in range(fine):
+        t = v.copy()
+        for k in range(1, 40):
+            t = (lo * np.r_[L(0), t[:-1]] + d * t + up * np.r_[t[1:], L(0)]) / (L(fine) * k)
+            v = v + t
+        v = v * np.exp(-c / fine)
+        big = max(big, np.abs(v).max())
+    return v, s, float(52 * EPS * s * math.exp((norm - float(c)) / s) * big), norm
+
+
+def birth_death(n, tau, augmented):
+    rng = np.random.default_rng(n)
+    b, d = rng.uniform(0.5, 2.0, n), rng.uniform(0.5, 2.0, n)
+    h = np.sqrt(b[:-1] * d[1:])  # the symmetric form of the section
+    lo, up, di = np.r_[0, h], np.r_[h, 0], -(b + d)
+    if augmented and n > 2:
+        di[-2:] = 0
+        up[-3:] = 0
+        lo[-1] = 1
+    return tau * lo, tau * di, tau * up
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 31, 32, 33, 64])
+@pytest.mark.parametrize("tau", [1e-9, 0.3, 5.0, 28.0])
+def test_sections(tri, n, tau):
+    T = birth_death(n, tau, augmented=True)
+    ref, s, bound, _ = column(*T)
+    ok, got = tri(*T)
+    assert ok and float(np.abs(got - ref).max()) <= bound
+
+
+@pytest.mark.parametrize("n", [8, 32])
+@pytest.mark.parametrize("tau", [1e-2, 0.3, 0.8])
+def test_last_rows_keep_their_size(tri, n, tau):
+    # a step's error estimate: row i starts with term i, norm^i / i! below it in size. Terms
+    # up to n + 8 leave less than norm^9 n! / (n + 8)! of the last row
+    T = birth_death(n, tau, augmented=False)
+    ref, s, _, norm = column(*T)
+    ok, got = tri(*T)
+    assert ok and s == 1
+    rest = norm ** 9 * math.factorial(n) / math.factorial(n + 8)
+    scale = math.exp(2 * norm)  # the shift's factor and the sum over the later terms
+    assert abs(float(got[-1] / ref[-1]) - 1) <= scale * (rest + 52 * EPS * n)
+
+
+@pytest.mark.parametrize("kind", ["zero", "nilpotent", "growing", "skew"])
+def test_other_matrices(tri, kind):
+    n = 17
+    z = np.zeros(n)
+    T = {"zero": (z, z, z), "nilpotent": (np.full(n, 11.0), z, z), "growing": (z + 0.5, z + 3.0, z + 0.25),
+         "skew": (np.full(n, 9.0), z, np.full(n, -9.0))}[kind]
+    T = tuple(np.array(v) for v in T)
+    T[0][0] = T[2][-1] = 0.0
+    ref, s, bound, _ = column(*T)
+    ok, got = tri(*T)
+    assert ok and float(np.abs(got - ref).max()) <= bound
+
+
+def test_declines(tri):
+    lo, di, up = birth_death(32, 1.0, augmented=False)
+    norm = column(lo, di, up)[3]
+    assert tri(*(255.0 / norm * v for v in (lo, di, up)))[0]
+    ok, out = tri(*(257.0 / norm * v for v in (lo, di, up)))
+    assert not ok and np.isnan(out).all()  # the caller takes the dense form
+    for bad in (np.nan, np.inf):
+        d = di.copy()
+        d[3] = bad
+        assert not tri(lo, d, up)[0]
