@@ -11,6 +11,7 @@ columns, and sink rows of 1 to 700 entries.
 """
 import numpy as np
 import pytest
+import scipy.linalg
 
 import models
 import numcme_hip as nh
@@ -111,3 +112,36 @@ def test_max_steps_leaves_the_state_reached(gpu):
     assert got[0][0] == got[1][0] > 0.0
     assert np.array_equal(got[0][1], got[1][1])
     assert abs(got[0][1].sum() - 1.0) < 1e-9
+
+
+@pytest.mark.parametrize("n,theta,tol", [(300, (0.05, 0.5, 15.0, 1.0), 1e-9), (700, (0.05, 0.5, 15.0, 1.0), 1e-6),
+                                         (700, (0.02, 0.2, 30.0, 0.5), 1e-6), (300, (0.5, 5.0, 100.0, 1.0), 1e-6)])
+def test_near_stationary_states(gpu, n, theta, tol):
+    # stiff boxes far above the law's support, run to ten relaxation times: the step's error
+    # estimate falls slowly with the step there, and the step control has to get by with its
+    # ten rejections
+    S, props, th = models.telegraph(theta)
+    states = np.asarray(models.telegraph_states(n - 1))
+    dt, K = 10.0, 20
+    N = 2 * n
+    G = np.zeros((N + 4, N + 4))
+    for j, (off, on, m) in enumerate(states.tolist()):
+        gene = (n + m, theta[0]) if off else (m, theta[1])
+        for i, rate in (gene, (j + 1 if m + 1 < n else N + 2, theta[2] * on), (j - 1, theta[3] * m)):
+            if rate:
+                G[i, j] += rate
+                G[j, j] -= rate
+    P = scipy.linalg.expm(G * dt)
+    ref = np.zeros(N + 4)
+    ref[n // 3 * 2], ref[0] = 0.75, 0.25
+    ts = dt * np.arange(K + 1)
+    model = nh.CmeModel(S, models.to_product(props), th)
+    space = nh.StateSpaceSparse(S, states)
+    A = nh.FspMatrixSparse(space, None, precision="fp64", model=model)
+    out = _integrate(A, nh.KrylovExpv(m=30, tol=tol, precision="fp64").opts(1e-6, 1e-4), ref, 0.0, ts, space)
+    for k in range(K + 1):
+        got = np.concatenate([out.p[k].values, out.sinks[k]])
+        # a step accepts 1.2 tol per unit time; the semigroup does not amplify it in the
+        # 1-norm, which 2-norm errors bound within sqrt(N)
+        assert np.linalg.norm(got - ref) <= 1.2 * tol * ts[k] * np.sqrt(N) + 1e-12
+        ref = P @ ref
