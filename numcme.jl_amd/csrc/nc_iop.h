@@ -169,11 +169,25 @@ __device__ inline void iop_group_sums(double (&t)[kIopSums], double* part, int g
   }
 }
 
-// Tail rows added to the totals, one after the other (x, x1, q of tail row r in sx, sx1, sq)
+// Tail rows added to the totals, one after the other (x, x1, q of tail row r in sx, sx1, sq,
+// arrays of kIopTail). Four rows' values are loaded together (a row at a time was an LDS
+// latency each); rows past the last weigh zero, which leaves a sum as it is.
 __device__ inline void iop_add_tail(int rows, const double* sx, const double* sx1, const double* sq,
                                     double (&tot)[kIopSums]) {
   double tl[kIopSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int r = 0; r < rows; ++r) iop_row_sums(sx[r], sx1[r], sq[r], tl);
+  for (int r = 0; r < rows; r += 4) {
+    double x[4], x1[4], q[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = r + u < kIopTail ? r + u : 0;
+      x[u] = sx[i], x1[u] = sx1[i], q[u] = sq[i];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool on = r + u < rows;  // the others may hold anything
+      iop_row_sums(on ? x[u] : 0.0, on ? x1[u] : 0.0, on ? q[u] : 0.0, tl);
+    }
+  }
 #pragma unroll
   for (int k = 0; k < kIopSums; ++k) tot[k] += tl[k];
 }

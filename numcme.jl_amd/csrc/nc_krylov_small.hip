@@ -32,21 +32,36 @@ struct alignas(2 * sizeof(T)) Two {
   T v[2];
 };
 
-__device__ inline double shfl_sum(double v) {  // the tree of the mat-vec's sink rows
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
+// The tree of the mat-vec's sink rows (lane l with l + 32, then 16, 8, 4, 2, 1; lane 0's sum)
+// by register permutes: the halves and the odd rows of 16 swapped, then rotations within a
+// row, whose lanes agree modulo the width already summed.
+__device__ inline double tree_sum(double v) {
+  auto swapped = [](auto pl, double x) {
+    const auto lo = pl((uint32_t)__double2loint(x)), hi = pl((uint32_t)__double2hiint(x));
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+  };
+  v = swapped([](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); }, v);
+  v = swapped([](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); }, v);
+  v = iop_dpp_add<0x128>(v);
+  v = iop_dpp_add<0x124>(v);
+  v = iop_dpp_add<0x122>(v);
+  return iop_dpp_add<0x121>(v);
 }
 
 // Thread t owns rows 512 p + 2 t, + 1 for p < P: their matrix entries stay in registers for
 // the whole process, the vector being multiplied lives in LDS, and a column is two barriers:
-// one before its gathers, one at its sums. Latency bound (about 0.7 us a column on 800
-// states: LDS gathers, the wave sums, one square root and one division), where the launches
-// of the process cost 5 us a column. KT: slots, entries past K weigh zero.
+// one before its gathers, one at its sums. Latency bound (LDS gathers, the wave sums, one
+// square root and one division): a column of 31 takes 1.9 us at 240 rows, 2.6 at 1,400 and
+// 3.4 at 3,000, where the launches of the process cost 5 us a column. H and the sink values
+// collect in LDS and go to the host's memory at the end, and nothing in the column loop is
+// indexed by a loop counter (private memory): a wait for either also waits for the stores
+// to host memory, 2.3, 3.0 and 4.4 us a column. KT: slots, entries past K weigh zero.
 template <typename VT, int KT, int P>
 __global__ __launch_bounds__(kT) void k_krylov_small(SmallArgs<VT> a) {
   __shared__ double s_x[kIopRows * P];
   __shared__ double s_w[kIopWaves][kIopSums];
   __shared__ double s_sv[3][kIopTail], s_sq[kIopTail];
+  __shared__ double s_k[32][4], s_ks[32][kIopTail], s_avn;  // for the host, written at the end
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = (int)a.n, R = a.R;
   double dg[P][2];
@@ -90,7 +105,7 @@ __global__ __launch_bounds__(kT) void k_krylov_small(SmallArgs<VT> a) {
   double x[P][2], x1[P][2], q[P][2];  // V_c, V_{c-1} and q_c of the thread's rows
   double usink = 0.0;
   if (a.nv >= 0) {
-    constexpr int C = 8;
+    constexpr int C = P <= 2 ? 16 : 8;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int i0 = kIopRows * p + 2 * tid, ic = i0 < n ? i0 : 0;
@@ -168,21 +183,24 @@ __global__ __launch_bounds__(kT) void k_krylov_small(SmallArgs<VT> a) {
 #pragma unroll
       for (int r = 0; r < 2; ++r) iop_row_sums(x[p][r], x1[p][r], q[p][r], t);  // rows past the states are zero
     // sink rows, one wave each, its entries in the order of the launches' 256 threads
-    for (int r = wave, j = 0; r < R; r += kIopWaves, ++j) {
-      const int64_t b0 = j < 2 ? e0[j & 1] : a.sink_off[r], b1 = j < 2 ? e1[j & 1] : a.sink_off[r + 1];
+    auto sink_row = [&](int r, int64_t b0, int64_t b1, bool kept, int src, double weight) {
       double s = 0.0;
       for (int v = 0; v < 4 && b0 + 64 * v < b1; ++v) {
         double acc = 0.0;
         int64_t e = b0 + 64 * v + lane;
-        if (v == 0 && j < 2) {
-          acc = __fma_rn(sw[j & 1], s_x[ss[j & 1]], acc);
+        if (v == 0 && kept) {
+          acc = __fma_rn(weight, s_x[src], acc);
           e += 256;
         }
         for (; e < b1; e += 256) acc = __fma_rn((double)a.sink_val[e], s_x[a.sink_src[e]], acc);
-        s += shfl_sum(acc);
+        s += tree_sum(acc);
       }
       if (lane == 0) s_sq[r] = s;
-    }
+    };
+    if (wave < R) sink_row(wave, e0[0], e1[0], true, ss[0], sw[0]);
+    if (wave + kIopWaves < R) sink_row(wave + kIopWaves, e0[1], e1[1], true, ss[1], sw[1]);
+    for (int r = wave + 2 * kIopWaves; r < R; r += kIopWaves)
+      sink_row(r, a.sink_off[r], a.sink_off[r + 1], false, 0, 0.0);
 #pragma unroll
     for (int k = 0; k < kIopSums; ++k) t[k] = iop_wave_sum(t[k]);
     if (lane == 0) {
@@ -198,19 +216,13 @@ __global__ __launch_bounds__(kT) void k_krylov_small(SmallArgs<VT> a) {
     iop_add_tail(R, sx, sx1, s_sq, tot);
     const IopCoef o = iop_coef(tot, c, scp, a.btol);
     if (tid == 0) {
-      if (c > 0)
-        a.host[L.H(c, c - 1)] = o.nrm;
-      else
-        a.host[L.misc(MISC_BETA)] = o.nrm;
-      a.host[L.sc(c)] = o.sc;
-      if (c < a.m) {
-        a.host[L.H(c, c)] = o.h1;
-        if (c > 0) a.host[L.H(c - 1, c)] = o.h0;
-      } else {
-        a.host[L.misc(MISC_AVN)] = o.sc * sqrt(tot[4]);
-      }
+      s_k[c][0] = o.nrm;
+      s_k[c][1] = o.sc;
+      s_k[c][2] = o.h1;
+      s_k[c][3] = o.h0;
+      if (c == a.m) s_avn = o.sc * sqrt(tot[4]);
     }
-    if (tid < R) a.host[L.sinkv(c, tid, R)] = sx[tid];
+    if (tid < R) s_ks[c][tid] = sx[tid];
     if (c == a.m) break;
     VT* vn = a.V + (int64_t)(c + 1) * a.Np;
 #pragma unroll
@@ -236,6 +248,19 @@ __global__ __launch_bounds__(kT) void k_krylov_small(SmallArgs<VT> a) {
     }
     scp = o.sc;
   }
+  __syncthreads();
+  if (tid <= a.m) {
+    const int c = tid;
+    a.host[c > 0 ? L.H(c, c - 1) : L.misc(MISC_BETA)] = s_k[c][0];
+    a.host[L.sc(c)] = s_k[c][1];
+    if (c < a.m) {
+      a.host[L.H(c, c)] = s_k[c][2];
+      if (c > 0) a.host[L.H(c - 1, c)] = s_k[c][3];
+    } else {
+      a.host[L.misc(MISC_AVN)] = s_avn;
+    }
+  }
+  for (int i = tid; i < (a.m + 1) * R; i += kT) a.host[L.sinkv(0, 0, R) + i] = s_ks[i / R][i % R];
 }
 
 template <typename VT>
