@@ -33,18 +33,18 @@ sys.path.insert(0, str(ROOT / "numcme.jl_amd"))
 
 HBM_PEAK_GBPS = 8000.0
 TRAFFIC_PROFILE = ROOT / "profiles" / "k_matvec_toggle1024_fp32.md"
-PROJECTION_PROFILE = ROOT / "profiles" / "k_matvec_projection_toggle1024_fp32.md"
+COLUMN_PROFILE = ROOT / "profiles" / "k_krylov_col_toggle1024_fp32.md"
 
 
-def measured_traffic(rows_per_thread, precision, matrix_free, projection=False):
+def measured_traffic(rows_per_thread, precision, matrix_free, column=False):
     """HBM bytes per mat-vec launch from the committed rocprofv3 counter runs (FETCH_SIZE
     plus WRITE_SIZE, calibrated on a copy kernel), for the mode and launch shape in use
-    (projection: the mat-vec with the Krylov projection epilogue, averaged over a solve's
-    launches); None when no counter run covers it."""
-    prof = PROJECTION_PROFILE if projection else TRAFFIC_PROFILE
+    (column: the launch that forms, multiplies and sums a Krylov basis vector); None when no
+    counter run covers it."""
+    prof = COLUMN_PROFILE if column else TRAFFIC_PROFILE
     if precision != "fp32" or not prof.exists():
         return None
-    mode = "projection" if projection else {0: "stored", 1: "computed_values", 2: "matrix_free"}[int(matrix_free)]
+    mode = "column" if column else {0: "stored", 1: "computed_values", 2: "matrix_free"}[int(matrix_free)]
     key = f"traffic_bytes_per_launch mode={mode} rows_per_thread={rows_per_thread}:"
     for line in prof.read_text().splitlines():
         if line.startswith(key):
@@ -696,11 +696,10 @@ def spmv_probe(nh, precision, reps):
             times[f"{names[mode]} rows_per_thread={rows}"] = A.bench_matvec(reps=reps) * 1e3
     A.set_matrix_free(default)
     A.set_rows_per_thread(2)
-    # the mat-vec with its Krylov projection epilogue over the basis sizes of one Krylov
-    # step at m = 30 (1..30 vectors for the columns, 1 for the norm of A v_m), reps
-    # launches each
-    proj = {nv: A.bench_projection(nv, reps=reps) * 1e3 for nv in range(1, 31)}
-    proj_step_mean = (sum(proj.values()) + proj[1]) / 31
+    # the launches of one Krylov step at m = 30 (basis vectors 1..31, the last for the norm
+    # of A v_m), reps each
+    column = {nv: A.bench_projection(nv, reps=reps) * 1e3 for nv in range(1, 32)}
+    column_step_mean = sum(column.values()) / 31
     x = torch.ones(64 * 1024 * 1024, dtype=torch.float32, device="cuda")  # 256 MiB
     y = torch.empty_like(x)
     for _ in range(3):
@@ -708,7 +707,7 @@ def spmv_probe(nh, precision, reps):
     torch.cuda.synchronize()
     info = A.info()
     print(json.dumps({"probe": "spmv", "precision": precision, "reps": reps, "mean_launch_us": times,
-                      "projection_mean_launch_us": proj, "projection_step_mix_mean_us": proj_step_mean,
+                      "column_mean_launch_us": column, "column_step_mean_us": column_step_mean,
                       "csr_bytes_per_matvec": info["csr_bytes_per_matvec"],
                       "own_bytes_per_matvec_default_mode": info["bytes_per_matvec"],
                       "copy_bytes_each_way": x.numel() * 4}), flush=True)
@@ -876,8 +875,8 @@ def main():
 
     # mat-vec roofline: one more solve with HIP events recorded around every mat-vec
     # launch on the solver's stream (graphs off, since events cannot sit inside them):
-    # mode 1 times the launches as the solves run them (the mat-vec with its projection
-    # epilogue), mode 2 the plain mat-vec (the projection sums then run as a separate pass)
+    # mode 1 times the launches as the solves run them (each forms, multiplies and sums a
+    # basis vector), mode 2 the plain mat-vec (vector and sums by launches of their own)
     def timed_solve(mode=1):
         tim = Solver(L, A, args.precision, mode, tol=args.krylov_tol)
         tim.set_state(u0)
@@ -888,18 +887,18 @@ def main():
             st["matvecs_timed"]
 
     mf_on = bool(info["matrix_free"])
-    # the stored generator at 2 rows per thread (the default shape) carries the epilogue
-    projection = not mf_on and info["rows_per_thread"] == 2
+    # the stored generator at 2 rows per thread (the default shape) has the column kernel
+    column = not mf_on and info["rows_per_thread"] == 2
     avg_mv_s, mv_n = timed_solve(1)
-    avg_plain_s, plain_n = timed_solve(2) if projection else (avg_mv_s, mv_n)
+    avg_plain_s, plain_n = timed_solve(2) if column else (avg_mv_s, mv_n)
     back_to_back_ms = A.bench_matvec(reps=200)
-    # the epilogue kernel back to back over one Krylov step's basis sizes (1..30, then 1)
-    proj_b2b_ms = ((sum(A.bench_projection(nv, reps=20) for nv in range(1, 31)) + A.bench_projection(1, reps=20)) / 31
-                   if projection else None)
-    # the projection epilogue reads the column's basis vectors V_0..V_j at the state rows:
-    # j + 1 = 1..m for the m columns and 1 for the norm of A v_m, m + 1 launches a step
+    # the column kernel back to back over one Krylov step's basis vectors
+    column_b2b_ms = sum(A.bench_projection(nv, reps=20) for nv in range(1, 32)) / 31 if column else None
+    # beyond a mat-vec's bytes (its input counts as the vector formed and stored) a column
+    # reads the previous product (FP64) and the two vectors before its own at the state rows,
+    # for all but the first of the m + 1 launches of a step
     m_k = 30
-    proj_bytes = (m_k * (m_k + 1) // 2 + 1) / (m_k + 1) * info["n_states"] * (4 if args.precision == "fp32" else 8)
+    column_bytes = m_k / (m_k + 1) * info["n_states"] * (8 + 2 * (4 if args.precision == "fp32" else 8))
     stored = None
     if mf_on:
         # the same kernel reading the stored generator, for comparison
@@ -913,9 +912,9 @@ def main():
         A.set_matrix_free(info["matrix_free"])
     rows_tuned, _ = A.autotune(reps=30)  # reported only: the timed solves use the default shape
     A.set_rows_per_thread(info["rows_per_thread"])
-    # the dominant kernel of the timed solves: the mat-vec with its projection epilogue
-    # (CSR-equivalent mat-vec bytes plus the basis vectors it reads), or the plain mat-vec
-    launch_bytes = info["csr_bytes_per_matvec"] + (proj_bytes if projection else 0.0)
+    # the dominant kernel of the timed solves: the column kernel (CSR-equivalent mat-vec
+    # bytes plus the product and the vectors it reads), or the plain mat-vec
+    launch_bytes = info["csr_bytes_per_matvec"] + (column_bytes if column else 0.0)
     achieved = launch_bytes / avg_mv_s / 1e9
     spmv_achieved = info["csr_bytes_per_matvec"] / avg_plain_s / 1e9
     line = {
@@ -955,24 +954,24 @@ def main():
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBPS,
-            "traffic": measured_traffic(info["rows_per_thread"], args.precision, info["matrix_free"], projection),
-            "traffic_source": (PROJECTION_PROFILE if projection else TRAFFIC_PROFILE).name,
-            "kernel": ("k_matvec with the Arnoldi projection epilogue (FSP SpMV, stored generator, plus the "
-                       "column's projection sums over 512-row blocks)" if projection else
+            "traffic": measured_traffic(info["rows_per_thread"], args.precision, info["matrix_free"], column),
+            "traffic_source": (COLUMN_PROFILE if column else TRAFFIC_PROFILE).name,
+            "kernel": ("k_krylov_col (FSP SpMV, stored generator, with the basis vector formed where it is "
+                       "gathered and the column's sums)" if column else
                        "k_matvec (FSP SpMV), " + ("computed values: off-diagonal values from per-reaction tables, "
                                                   "columns from row offsets, the FP64 diagonal read; achieved "
                                                   "counts the CSR-equivalent bytes" if mf_on else "stored generator")),
             "bytes_per_launch": launch_bytes,
             "bytes_per_launch_csr": info["csr_bytes_per_matvec"],
-            "bytes_per_launch_projection": proj_bytes if projection else 0.0,
+            "bytes_per_launch_vectors": column_bytes if column else 0.0,
             "bytes_per_launch_own_layout": info["bytes_per_matvec"],
             "stored_generator": stored,
             "avg_launch_us": avg_mv_s * 1e6,
             "launches_timed": mv_n,
-            "back_to_back_step_mix_launch_us": proj_b2b_ms * 1e3 if projection else None,
+            "back_to_back_step_mix_launch_us": column_b2b_ms * 1e3 if column else None,
             "spmv": {
-                "kernel": "k_matvec (FSP SpMV), stored generator, timed in a solve whose projection sums run as "
-                          "a separate pass" if projection else "as above",
+                "kernel": "k_matvec (FSP SpMV), stored generator, timed in a solve whose vectors and sums are "
+                          "launches of their own" if column else "as above",
                 "avg_launch_us": avg_plain_s * 1e6,
                 "launches_timed": plain_n,
                 "achieved_csr_equivalent": spmv_achieved,

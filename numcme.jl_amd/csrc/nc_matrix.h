@@ -83,7 +83,7 @@ struct nc_matrix_s {
   int64_t nnz_ref = 0, n_sink_entries = 0;
   double norm1 = 0.0;
   // kernel timing (HIP events around mat-vec launches); timing_plain: the launches timed
-  // are plain mat-vecs (the Krylov projection sums then run as a separate pass)
+  // are plain mat-vecs (a Krylov column's vector and sums then are launches of their own)
   bool timing = false;
   bool timing_plain = false;
   std::vector<hipEvent_t> ev;

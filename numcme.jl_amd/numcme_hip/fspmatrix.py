@@ -122,8 +122,8 @@ class FspMatrixSparse(L.Handle):
         return ms.value
 
     def bench_projection(self, nv, reps=100):
-        """Mean time in ms of the Krylov mat-vec with its projection epilogue over nv basis
-        vectors (HIP events on the matrix stream)."""
+        """Mean time in ms of the launch that forms, multiplies and sums basis vector nv of
+        the Krylov process (HIP events on the matrix stream)."""
         ms = C.c_double()
         L.call("nc_matrix_bench_projection", self.handle, int(nv), int(reps), C.byref(ms))
         return ms.value

@@ -30,10 +30,10 @@ class KrylovExpv:
     tol: float = 1e-12
     precision: str = "fp64"
     # HIP events around every mat-vec launch: 1 (or True) as the solve runs them (the
-    # mat-vec with its projection epilogue where the generator has one), 2 plain mat-vecs
-    # (the projection sums then run as a separate pass; same results)
+    # launch that forms, multiplies and sums a basis vector where the generator has one), 2
+    # plain mat-vecs (the vector and its sums by launches of their own; same results)
     time_kernels: int = 0
-    graphs: bool = True  # replay each Arnoldi process as a captured HIP graph
+    graphs: bool = True  # replay each Krylov process as a captured HIP graph
 
     def opts(self, odeatol, odertol):
         o = L.nc_solve_opts()
