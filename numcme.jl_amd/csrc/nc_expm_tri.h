@@ -36,8 +36,10 @@ inline bool expm_tri(int n, const double* lo, const double* di, const double* up
     norm = s > norm ? s : norm;
   }
   int parts = 1;
-  while (norm > kTriPart * parts || norm - c > kTriExcess * parts) parts *= 2;
-  if (parts > max_parts) return false;
+  while (norm > kTriPart * parts || norm - c > kTriExcess * parts) {
+    if (parts > max_parts / 2) return false;
+    parts *= 2;
+  }
   const double scale = 1.0 / parts, part = norm * scale, damp = std::exp(-c * scale);
   // up to the first term below 2^-57, and at least 8 terms into the last row, which term
   // n - 1 reaches first: the step's error estimate is the last rows, however small

@@ -128,3 +128,16 @@ def test_declines(tri):
         d = di.copy()
         d[3] = bad
         assert not tri(lo, d, up)[0]
+
+
+def test_declines_large_growth(tri):
+    # nearly equal positive diagonal entries: the shift takes them out of the norm, and the
+    # number of parts goes by e^{-c} alone, past any power of two that an int holds
+    n = 5
+    z = np.zeros(n)
+    for d in (2e10, 1e300):
+        ok, out = tri(z, np.full(n, d), z)
+        assert not ok and np.isnan(out).all()
+    # 32 parts of excess 4 are the most that the form takes
+    assert tri(z, np.full(n, 127.0), z)[0]
+    assert not tri(z, np.full(n, 129.0), z)[0]
