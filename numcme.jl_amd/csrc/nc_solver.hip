@@ -585,6 +585,8 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
       }
     }
     const double avnorm = hb[L.misc(MISC_AVN)];
+    const double floor_err = krylov_floor(S) * beta;
+    auto allowed = [&](double tau) { return std::max(tau * tol, floor_err); };  // error of a step tau
     const int mxf = mb + k1;  // size of the exponentiated matrix
     std::vector<double> F(mxf);  // first column of exp(tau H), H tridiagonal
     auto exp_tau = [&](double tau, std::vector<double>& out) {
@@ -616,13 +618,13 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
         err_loc = phi1;
         xm = 1.0 / (m - 1);
       }
-      if (err_loc <= delta * t_step * tol) break;
+      if (err_loc <= delta * allowed(t_step)) break;
       if (ireject == mxrej) throw Error(NC_ERR_NUMERIC, "Krylov step rejected too many times; tolerance too tight");
       // the step that the estimate's order asks for; from the second rejection on at most half:
       // near a stationary state of a stiff generator the estimate falls like tau, not
       // tau^m, and shrinking by a tenth each time used up the rejections (an exponential
       // costs 6 us, a step a hundred and more)
-      const double fac = gamma * std::pow(t_step * tol / err_loc, xm);
+      const double fac = gamma * std::pow(allowed(t_step) / err_loc, xm);
       t_step = round_step(t_step * (ireject > 0 ? std::min(fac, 0.5) : fac));
       S->st.rejected++;
     }
@@ -669,7 +671,7 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
     S->st.steps++;
     err_loc = std::max(err_loc, 1e-300);
     S->st.error_estimate += std::max(err_loc, S->anorm * 2.220446049250313e-16);
-    if (k1 != 0 && !fire) S->t_new = round_step(gamma * t_step * std::pow(t_step * tol / err_loc, xm));
+    if (k1 != 0 && !fire) S->t_new = round_step(gamma * t_step * std::pow(allowed(t_step) / err_loc, xm));
     if (fire) {
       ev->fired = true;
       break;

@@ -114,6 +114,62 @@ def test_max_steps_leaves_the_state_reached(gpu):
     assert abs(got[0][1].sum() - 1.0) < 1e-9
 
 
+def _telegraph_exact(n, theta, dt, K):
+    """Exact states at K + 1 times of the box of n counts, from a distribution on two states,
+    and how much the exponential amplifies an error in the 2-norm over that time: at most, and
+    in the mean square over errors of independent entries."""
+    states = np.asarray(models.telegraph_states(n - 1))
+    N = 2 * n
+    G = np.zeros((N + 4, N + 4))
+    for j, (off, on, m) in enumerate(states.tolist()):
+        gene = (n + m, theta[0]) if off else (m, theta[1])
+        for i, rate in (gene, (j + 1 if m + 1 < n else N + 2, theta[2] * on), (j - 1, theta[3] * m)):
+            if rate:
+                G[i, j] += rate
+                G[j, j] -= rate
+    E, s, amp, rms = scipy.linalg.expm(G * (dt / 16)), dt / 16, 1.0, 1.0
+    while True:
+        amp, rms = max(amp, np.linalg.norm(E, 2)), max(rms, np.linalg.norm(E) / np.sqrt(N))
+        if s == dt:
+            P = E
+        if s >= dt * K:
+            break
+        E, s = E @ E, 2 * s
+    u = np.zeros(N + 4)
+    u[n // 3 * 2], u[0] = 0.75, 0.25
+    ref = [u]
+    for _ in range(K):
+        ref.append(P @ ref[-1])
+    return states, ref, amp, rms
+
+
+def _telegraph_solve(n, theta, dt, K, tol, precision):
+    states, ref, amp, rms = _telegraph_exact(n, theta, dt, K)
+    S, props, th = models.telegraph(theta)
+    model = nh.CmeModel(S, models.to_product(props), th)
+    space = nh.StateSpaceSparse(S, states)
+    A = nh.FspMatrixSparse(space, None, precision=precision, model=model)
+    ts = dt * np.arange(K + 1)
+    out = _integrate(A, nh.KrylovExpv(m=30, tol=tol, precision=precision).opts(1e-6, 1e-4), ref[0], 0.0, ts, space)
+    err = [np.linalg.norm(np.concatenate([p.values, s]) - r) for p, s, r in zip(out.p, out.sinks, ref)]
+    return out.stats["steps"], ts, np.array(err), amp, rms * max(np.linalg.norm(r) for r in ref[1:])
+
+
+@pytest.mark.parametrize("n", [120, 300])
+def test_fp32_near_stationary_steps(gpu, n):
+    # Rates that FP32 holds exactly, ten relaxation times past the transient: what is left for
+    # a step to follow is the rounding of its first vector, 2^-24 of each entry at most, and
+    # asking for less than a quarter of that takes no more steps (1e-12 took 1.4 times the
+    # steps of 1e-9). The errors of the steps add up as a random walk: four deviations
+    theta = (0.0625, 0.5, 15.0, 1.0)
+    steps = {}
+    for tol in (1e-9, 1e-12):
+        steps[tol], ts, err, _, size = _telegraph_solve(n, theta, 10.0, 20, tol, "fp32")
+        k = steps[tol]
+        assert err.max() <= 4 * np.sqrt(k) * 2.0 ** -24 * size
+    assert steps[1e-12] <= 1.1 * steps[1e-9]
+
+
 @pytest.mark.parametrize("n,theta,tol", [(300, (0.05, 0.5, 15.0, 1.0), 1e-9), (700, (0.05, 0.5, 15.0, 1.0), 1e-6),
                                          (700, (0.02, 0.2, 30.0, 0.5), 1e-6), (300, (0.5, 5.0, 100.0, 1.0), 1e-6)])
 def test_near_stationary_states(gpu, n, theta, tol):
