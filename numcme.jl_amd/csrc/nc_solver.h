@@ -88,10 +88,11 @@ inline double krylov_breakdown_tol(const nc_solver_s* S) {
 // off by about 2^-25 of its norm to begin with. Steps that followed the estimate further down
 // resolved that rounding: near the stationary state of a telegraph box of 300 counts a
 // tolerance of 1e-9 took 1,181 steps (93 ms) and 1e-12 1,659 (128 ms), now 765 (61 ms) and 784
-// (62 ms) at the same error of 8e-9. Not below 12 vectors, where the steps are many and their truncation, unlike
-// the rounding, does not average out (three vectors: 3e-9 of error would become 2e-7).
+// (62 ms) at the same error of 8e-9. Not below 12 vectors, where the steps are many and their
+// truncation, unlike the rounding, does not average out (three vectors: 3e-9 of error would
+// become 2e-7), and not for sensitivities, whose norm says nothing of the rounding of p.
 inline double krylov_floor(const nc_solver_s* S) {
-  return S->vs == 4 && S->m >= 12 ? 0x1p-26 : 0.0;
+  return S->vs == 4 && S->m >= 12 && !S->SA ? 0x1p-26 : 0.0;
 }
 // Advance to t_target (or to the budget crossing when ev is given); with one_step the
 // call returns after the first accepted step.
