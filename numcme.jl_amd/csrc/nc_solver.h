@@ -1,6 +1,8 @@
 // Time integrators (internal): device-resident Krylov expv and Dormand-Prince 5(4).
 #pragma once
 
+#include <algorithm>
+#include <cmath>
 #include <memory>
 
 #include "nc_sens.h"
@@ -77,12 +79,26 @@ struct EventSpec {
 // and sink rows go to hbuf.
 bool krylov_small_fits(const nc_solver_s* S);
 void krylov_small_launch(nc_solver_s* S, int nv, double cu, const double* cs);
-// Happy breakdown: the residual of the exhausted space is |beta| h per unit time, so h has to
-// fall below the tolerance the caller asks for, per unit time too (Expokit's fixed 1e-7
-// let a solve near its stationary state jump to the next output with 1e-6 of error).
-inline double krylov_breakdown_tol(const nc_solver_s* S) {
+// Error per unit time that a step's estimate is held to. With full orthogonalisation the
+// error lay two to three orders below the estimate, with two vectors it comes near it: held to
+// the tolerance itself, FP64 errors grew by up to a thousand times (telegraph box of 120
+// counts over 200 time units at 1e-9: full 49 steps, 6.5e-12; two vectors 63 steps, 2.5e-9).
+// 10^(-m/10) of it makes every step a fifth shorter whatever m is, and the errors are the full
+// form's or less (78 steps, 1.0e-13; sweep of 42 FP64 solves at 1e-9 and 1e-12: none above
+// it). Not below 1e-14, where the estimate is rounding.
+inline double krylov_step_tol(const nc_solver_s* S) {
   const double tol = S->opts.krylov_tol;
-  return tol < 1e-14 ? 1e-14 : (tol < 1e-7 ? tol : 1e-7);
+  return std::max(tol * std::pow(10.0, -0.1 * S->m), std::min(tol, 1e-14));
+}
+// Happy breakdown: the residual of the exhausted space is |beta| h per unit time, so h has to
+// fall below the tolerance the caller asks for, per unit time too (Expokit's fixed 1e-7 let
+// solves near a stationary state jump to the next output with 2e-5 of error). In FP64 storage
+// a tenth of it: that jump is most of the error there (300 counts at 1e-6: 1.7e-5 became
+// 1.7e-6 with 28% more steps, the step tolerance above included). In FP32 h does not fall much
+// below 1e-7, and a smaller threshold costs four times the steps.
+inline double krylov_breakdown_tol(const nc_solver_s* S) {
+  const double tol = std::min(S->opts.krylov_tol, 1e-7) * (S->vs == 8 ? 0.1 : 1.0);
+  return std::max(tol, 1e-14);
 }
 // Error that a step need not go below, relative to |V_0|: the first vector rounded to FP32 is
 // off by about 2^-25 of its norm to begin with. Steps that followed the estimate further down

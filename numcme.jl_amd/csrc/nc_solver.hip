@@ -516,7 +516,7 @@ void krylov_advance(nc_solver_s* S, double t_target, EventSpec* ev, bool one_ste
   const int R = A->nr;
   hipStream_t s = S->s;
   const bool fp32 = A->precision == NC_FP32;
-  const double tol = S->opts.krylov_tol;
+  const double tol = krylov_step_tol(S);
   const double btol = krylov_breakdown_tol(S), gamma = 0.9, delta = 1.2;
   const int mxrej = 10;
   if (!S->started) {

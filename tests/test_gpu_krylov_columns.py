@@ -170,6 +170,16 @@ def test_fp32_near_stationary_steps(gpu, n):
     assert steps[1e-12] <= 1.1 * steps[1e-9]
 
 
+@pytest.mark.parametrize("n,theta,tol", [(120, (0.05, 0.1, 5.0, 0.05), 1e-6), (120, (0.05, 0.1, 5.0, 0.05), 1e-9),
+                                         (400, (0.05, 0.1, 5.0, 0.05), 1e-9), (300, (0.01, 0.01, 3.0, 0.02), 1e-9),
+                                         (400, (0.01, 0.01, 3.0, 0.02), 1e-6)])
+def test_fp64_errors(gpu, n, theta, tol):
+    # boxes whose Krylov space is never exhausted: at 30 vectors a step's error estimate is
+    # held to 1.2e-3 of the tolerance per unit time; 2e-13 for the roundings of the steps
+    _, ts, err, amp, _ = _telegraph_solve(n, theta, 10.0, 20, tol, "fp64")
+    assert (err <= amp * 1.2e-3 * tol * ts + 2e-13).all()
+
+
 @pytest.mark.parametrize("n,theta,tol", [(300, (0.05, 0.5, 15.0, 1.0), 1e-9), (700, (0.05, 0.5, 15.0, 1.0), 1e-6),
                                          (700, (0.02, 0.2, 30.0, 0.5), 1e-6), (300, (0.5, 5.0, 100.0, 1.0), 1e-6)])
 def test_near_stationary_states(gpu, n, theta, tol):
