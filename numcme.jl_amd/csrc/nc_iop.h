@@ -38,12 +38,12 @@ constexpr int kIopRows = 2 * kIopThreads;  // rows per block
 constexpr int kIopGroups = 512;  // workgroups of a column at most: every workgroup of the next
                                  // column folds their partials itself, 20 KB from L2 (1,024
                                  // groups: 2 us more a column)
-constexpr int kIopSmallBlocks = 4096 / kIopRows;  // up to here one group holds every block
 constexpr int kIopSums = 5;
 constexpr int kIopTail = 32;  // sink rows at most
 
-inline int iop_groups(int64_t nblk) {
-  if (nblk <= kIopSmallBlocks) return 1;
+// one: the one-workgroup process holds a space of this shape, and every form sums in its order
+inline int iop_groups(int64_t nblk, bool one) {
+  if (one) return 1;
   return nblk < kIopGroups ? (int)nblk : kIopGroups;
 }
 

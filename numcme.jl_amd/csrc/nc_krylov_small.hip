@@ -303,12 +303,11 @@ void launch_t(nc_solver_s* S, int nv, double cu, const double* cs) {
 }  // namespace
 
 // One workgroup is faster than a launch per column while a column's work on one CU stays
-// under a launch's latency; at most 16 rows a thread hold their matrix entries in registers
-// (8 with more than four slots).
+// under a launch's latency.
 bool krylov_small_fits(const nc_solver_s* S) {
   const nc_matrix_s* A = S->A;
   return !S->SA && !A->timing && A->mf_mode == 0 && A->tv_r.empty() && A->n_chunks == 0 && A->nr <= kIopTail &&
-         A->n >= 1 && A->K >= 1 && A->K <= 8 && A->n <= (A->K <= 4 ? 8 : 4) * kIopRows;
+         krylov_small_shape(A);
 }
 
 void krylov_small_launch(nc_solver_s* S, int nv, double cu, const double* cs) {

@@ -156,6 +156,13 @@ void matvec_launch_err(nc_matrix_s* A, double t, const void* v, double* out, hip
 // sums kernels.
 bool matvec_krylov_fusable(const nc_matrix_s* A);
 void matvec_launch_krylov(nc_matrix_s* A, hipStream_t s, const IopArgs& p);
+// Shapes that the one-workgroup process takes: at most 16 rows a thread hold their matrix
+// entries in registers (8 with more than four slots). Column sums of such a space are one
+// workgroup's in every form, so that all give the same bits; other spaces spread their blocks
+// (twelve slots on 3,375 FP64 states, one workgroup a column: 7.1 ms a solve, seven 2.5).
+inline bool krylov_small_shape(const nc_matrix_s* A) {
+  return A->n >= 1 && A->K >= 1 && A->K <= 8 && A->n <= (A->K <= 4 ? 8 : 4) * kIopRows;
+}
 // V_c over every row (the form kernel)
 void krylov_form(const IopArgs& p, bool fp32, hipStream_t s);
 // When kernel timing is on, hand out the next pair of HIP events for a dispatch-stamped

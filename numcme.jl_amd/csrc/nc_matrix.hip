@@ -2147,7 +2147,7 @@ double bench_projection(nc_matrix_s* A, int nv, int reps) {
   p.tail1 = A->n_rows;
   p.ld = Np;
   p.nblk = (A->n + kIopRows - 1) / kIopRows;
-  p.groups = iop_groups(p.nblk);
+  p.groups = iop_groups(p.nblk, krylov_small_shape(A));
   p.c = nv - 1;
   p.V = V.p;
   p.L = KLayout{31};

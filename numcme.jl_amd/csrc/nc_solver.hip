@@ -361,7 +361,7 @@ void solver_reduce_setup(nc_solver_s* S) {
   // sensitivity system sums every padded row
   S->kn = S->SA ? S->Np : S->A->n;
   S->kblk = std::max<int64_t>((S->kn + kIopRows - 1) / kIopRows, 1);
-  S->kgroups = iop_groups(S->kblk);
+  S->kgroups = iop_groups(S->kblk, !S->SA && krylov_small_shape(S->A));
   S->partials.reserve(std::max<size_t>(S->red_blocks, (size_t)2 * kIopSums * S->kgroups));
   if (!S->hpart) {
     // partials (up to kMaxRedBlocks, or one per row workgroup and sink row of the mat-vec's

@@ -69,7 +69,8 @@ def test_toggle_boxes(gpu, precision, box, order):
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
 @pytest.mark.parametrize("levels", [11, 12, 13, 40])
 def test_cascade_expanded(gpu, precision, levels):
-    # six slots: the one-workgroup form holds 2,048 states; expansion order, mixed columns
+    # six slots: the one-workgroup form holds 2,048 states, larger spaces spread their blocks
+    # over workgroups; expansion order, mixed columns
     S, props, th = models.cascade()
     space = nh.StateSpaceSparse(S, [0, 0, 0])
     space.expand(levels + 6)
@@ -79,7 +80,7 @@ def test_cascade_expanded(gpu, precision, levels):
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
 @pytest.mark.parametrize("bounds", [(8, 8, 8), (16, 17, 18)])
 def test_twelve_slots(gpu, precision, bounds):
-    # more slots than the fixed-count kernels
+    # more slots than the fixed-count kernels and the one-workgroup form: 2 and 12 blocks
     S, props, th = models.twelve_slot()
     _check(S, models.box_states(bounds), props, th, precision, (0.0, 0.2, 0.5))
 
