@@ -196,10 +196,11 @@ int nc_matrix_export(nc_matrix A, double t, int64_t* nnz, int64_t* rows, int64_t
  * stored-precision input, FP64 output) and report the mean kernel duration from HIP events
  * on the matrix's stream. No reference counterpart. */
 int nc_matrix_bench_matvec(nc_matrix A, double t, int32_t reps, double* mean_ms);
-/* The same for the launch that the Krylov integrator makes for basis vector nv (1..32): the
- * vector formed from the previous column's product and its two predecessors, the mat-vec
- * and the column's sums (the first vector is read, not formed). NC_ERR_UNSUPPORTED for
- * generators without that form. No reference counterpart. */
+/* The same for what the Krylov integrator launches for basis vector nv (1..32): the vector
+ * formed from the previous column's product and its two predecessors, the mat-vec and the
+ * column's sums (the first vector is read, not formed), one launch, or three where a sink
+ * row has more than 8,192 entries. NC_ERR_UNSUPPORTED for generators without that form. No
+ * reference counterpart. */
 int nc_matrix_bench_projection(nc_matrix A, int32_t nv, int32_t reps, double* mean_ms);
 /* Computed mat-vecs. A generator on a box state space in lattice order (species 0 fastest,
  * at most 4 species, at most 8 distinct stoichiometries with at most 4 reactions each)

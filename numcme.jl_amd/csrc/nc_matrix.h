@@ -163,8 +163,9 @@ void matvec_launch_krylov(nc_matrix_s* A, hipStream_t s, const IopArgs& p);
 inline bool krylov_small_shape(const nc_matrix_s* A) {
   return A->n >= 1 && A->K >= 1 && A->K <= 8 && A->n <= (A->K <= 4 ? 8 : 4) * kIopRows;
 }
-// V_c over every row (the form kernel)
+// V_c over every row, and the column's sums from the stored V_c and q_c (nc_solver.hip)
 void krylov_form(const IopArgs& p, bool fp32, hipStream_t s);
+void krylov_sums(const IopArgs& p, bool fp32, hipStream_t s);
 // When kernel timing is on, hand out the next pair of HIP events for a dispatch-stamped
 // launch (the caller increments ev_used after the launch); false when timing is off.
 bool matvec_timing_slot(nc_matrix_s* A, hipEvent_t* e0, hipEvent_t* e1);

@@ -2120,9 +2120,10 @@ double bench_matvec(nc_matrix_s* A, double t, int reps) {
   return ms / reps;
 }
 
-// Mean duration of the Krylov process's column kernel at basis vector nv (device-resident
-// zero vectors in the solver's padded layout), launched reps times back to back on the
-// matrix's stream.
+// Mean duration of a Krylov column at basis vector nv (device-resident zero vectors in the
+// solver's padded layout), launched reps times back to back on the matrix's stream: the
+// column kernel, or the form, mat-vec and sums launches where the sink rows are cut into
+// chunks.
 double bench_projection(nc_matrix_s* A, int nv, int reps) {
   const bool was = A->timing, was_plain = A->timing_plain;
   A->timing = false;
@@ -2135,9 +2136,11 @@ double bench_projection(nc_matrix_s* A, int nv, int reps) {
       A->timing_plain = p;
     }
   } restore{A, was, was_plain};
-  if (!matvec_krylov_fusable(A))
+  const bool fused = matvec_krylov_fusable(A);
+  const bool chunked = A->n_chunks > 0 && A->mf_mode == 0 && A->rows_per_thread == 2 && A->tv_r.empty() && A->K >= 1;
+  if (!fused && !chunked)
     throw Error(NC_ERR_UNSUPPORTED, "this generator's mat-vec has no Krylov column form (it needs the stored "
-                                    "generator, 2 rows per thread, short sink rows, no time-varying reactions)");
+                                    "generator, 2 rows per thread, no time-varying reactions)");
   NC_REQUIRE(nv >= 1 && nv <= 32, NC_ERR_ARG, "nv must be in 1..32");
   hipStream_t s = A->stream.s;
   const int64_t Np = (A->n_rows + 1023) / 1024 * 1024;
@@ -2162,12 +2165,22 @@ double bench_projection(nc_matrix_s* A, int nv, int reps) {
   NC_CHECK_HIP(hipMemsetAsync(q.p, 0, sizeof(double) * q.n, s));
   NC_CHECK_HIP(hipMemsetAsync(part.p, 0, sizeof(double) * part.n, s));
   NC_CHECK_HIP(hipMemsetAsync(kb.p, 0, sizeof(double) * kb.n, s));
-  matvec_launch_krylov(A, s, p);  // warm-up
+  const bool fp32 = A->precision == NC_FP32;
+  auto column = [&] {
+    if (fused) {
+      matvec_launch_krylov(A, s, p);
+      return;
+    }
+    if (p.c > 0) krylov_form(p, fp32, s);
+    matvec_launch(A, 0.0, V.p + (size_t)p.c * Np * A->vsize, p.q[p.c & 1], false, s, true);
+    krylov_sums(p, fp32, s);
+  };
+  column();  // warm-up
   hipEvent_t e0, e1;
   NC_CHECK_HIP(hipEventCreate(&e0));
   NC_CHECK_HIP(hipEventCreate(&e1));
   NC_CHECK_HIP(hipEventRecord(e0, s));
-  for (int k = 0; k < reps; ++k) matvec_launch_krylov(A, s, p);
+  for (int k = 0; k < reps; ++k) column();
   NC_CHECK_HIP(hipEventRecord(e1, s));
   NC_CHECK_HIP(hipEventSynchronize(e1));
   float ms = 0.f;

@@ -351,6 +351,14 @@ double round_step(double x) {
 
 }  // namespace
 
+void krylov_sums(const IopArgs& p, bool fp32, hipStream_t s) {
+  if (fp32)
+    k_krylov_sums<float><<<(unsigned)p.groups, kIopThreads, 0, s>>>(p);
+  else
+    k_krylov_sums<double><<<(unsigned)p.groups, kIopThreads, 0, s>>>(p);
+  NC_CHECK_HIP(hipGetLastError());
+}
+
 void solver_reduce_setup(nc_solver_s* S) {
   // Grid of the vector passes: 1024 blocks of 256 threads for a Krylov basis stored in
   // FP32 and 512 otherwise (on the 1024^2 toggle-switch solve, 256 to 4096 blocks are
@@ -428,8 +436,7 @@ static void krylov_process(nc_solver_s* S) {
     }
     if (c > 0) krylov_form(p, S->vs == 4, S->s);
     op_apply(S, 0.0, S->V.p + (size_t)c * S->Np * S->vs, p.q[c & 1]);
-    k_krylov_sums<BT><<<(unsigned)S->kgroups, kIopThreads, 0, S->s>>>(p);
-    NC_CHECK_HIP(hipGetLastError());
+    krylov_sums(p, S->vs == 4, S->s);
   }
   k_krylov_last<BT><<<1, kIopThreads, 0, S->s>>>(p, S->m, S->u.p, S->A->n, S->A->nr, S->hbuf_dev);
   NC_CHECK_HIP(hipGetLastError());

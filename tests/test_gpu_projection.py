@@ -81,6 +81,11 @@ def test_bench_projection(gpu):
         A.bench_projection(4, reps=1)
     A.set_matrix_free(0)
     assert A.bench_projection(2, reps=1) > 0.0
+    # sink rows of 9,001 entries, which the mat-vec reduces in chunks
+    space = nh.StateSpaceSparse(S, models.box_states([9000, 1]))
+    A = nh.FspMatrixSparse(space, models.to_product(props), th, precision="fp32")
+    for nv in (1, 2, 32):
+        assert A.bench_projection(nv, reps=3) > 0.0
 
 
 def test_large_space_grid_stride_pass(gpu):
