@@ -151,9 +151,9 @@ int64_t matvec_err_parts(const nc_matrix_s* A);  // row workgroups + sink rows
 void matvec_launch_err(nc_matrix_s* A, double t, const void* v, double* out, hipStream_t s, const RkErrEpilogue& epi);
 // One column of the Krylov process (nc_iop.h) in one launch: V_c formed from q_{c-1} and the
 // two vectors before it while the mat-vec gathers it, q_c = A V_c and the column's sums.
-// Stored time-invariant generators at 2 rows per thread whose sink rows are not cut into
-// chunks, unless plain mat-vecs are being timed; other generators take the form / mat-vec /
-// sums kernels.
+// Stored time-invariant generators whose sink rows are not cut into chunks, unless plain
+// mat-vecs are being timed; other generators take the form / mat-vec / sums kernels. The
+// mat-vec's rows per thread do not matter to it: it has its own split.
 bool matvec_krylov_fusable(const nc_matrix_s* A);
 void matvec_launch_krylov(nc_matrix_s* A, hipStream_t s, const IopArgs& p);
 // Shapes that the one-workgroup process takes: at most 16 rows a thread hold their matrix

@@ -2014,8 +2014,8 @@ void krylov_form(const IopArgs& p, bool fp32, hipStream_t s) {
 }
 
 bool matvec_krylov_fusable(const nc_matrix_s* A) {
-  return A->mf_mode == 0 && A->rows_per_thread == 2 && !(A->timing && A->timing_plain) && A->tv_r.empty() &&
-         A->K >= 1 && A->n >= 1 && A->n_chunks == 0;
+  return A->mf_mode == 0 && !(A->timing && A->timing_plain) && A->tv_r.empty() && A->K >= 1 && A->n >= 1 &&
+         A->n_chunks == 0;
 }
 
 void matvec_launch_krylov(nc_matrix_s* A, hipStream_t s, const IopArgs& p) {
@@ -2137,10 +2137,10 @@ double bench_projection(nc_matrix_s* A, int nv, int reps) {
     }
   } restore{A, was, was_plain};
   const bool fused = matvec_krylov_fusable(A);
-  const bool chunked = A->n_chunks > 0 && A->mf_mode == 0 && A->rows_per_thread == 2 && A->tv_r.empty() && A->K >= 1;
+  const bool chunked = A->n_chunks > 0 && A->mf_mode == 0 && A->tv_r.empty() && A->K >= 1;
   if (!fused && !chunked)
     throw Error(NC_ERR_UNSUPPORTED, "this generator's mat-vec has no Krylov column form (it needs the stored "
-                                    "generator, 2 rows per thread, no time-varying reactions)");
+                                    "generator, no time-varying reactions)");
   NC_REQUIRE(nv >= 1 && nv <= 32, NC_ERR_ARG, "nv must be in 1..32");
   hipStream_t s = A->stream.s;
   const int64_t Np = (A->n_rows + 1023) / 1024 * 1024;
