@@ -1116,7 +1116,8 @@ void dispatch_r(int R, int K, const LaunchCfg& c, const MatArgs<VT>& a, const VT
     dispatch_k<VT, OT, 1>(K, c, a, vv, oo, acc);
 }
 
-// The launch arguments every mat-vec form shares, at time t.
+// The launch arguments every mat-vec form shares, at time t: joint values from the set that
+// holds that time (matrix_prepare_times), else the matrix's own.
 template <typename VT>
 MatArgs<VT> mat_args(const nc_matrix_s* A, double t) {
   MatArgs<VT> a{};
@@ -1694,7 +1695,7 @@ void joint_refresh(nc_matrix_s* A, double t) {
   if (t != A->t_cache && any_joint(A)) joint_fill<VT>(A, 0, 1, &t);
 }
 
-// Values at time t in some set, for a mat-vec that takes its arrays by joint_set_at
+// Values at time t in some set, for a mat-vec whose arguments (mat_args) take them from there
 template <typename VT>
 void joint_ready(nc_matrix_s* A, double t) {
   for (const auto& js : A->joint_sets)
