@@ -217,7 +217,12 @@ __global__ void k_connect_new(const uint32_t* table, uint64_t mask, const int32_
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallCands = 4096;
 constexpr int kSmallPer = kSmallCands / kSmallThreads;
-constexpr int64_t kSmallStates = int64_t(1) << 22;  // larger spaces are not grown for a few candidates
+// A level costs a few dependent reads of the table per candidate and thread: an L2's latency
+// up to here, beyond it memory's (the table of 2^20 states is 8 MB, an XCD's L2 holds 4).
+// One workgroup against the launches, us a level: 30 and 68 on 251,000 states (501
+// candidates), 75 and 90 on 501,000 (4,036), 60 and 64 on 1.0 million (1,001), 131 and 70 on
+// 2.0 million (1,401). Candidates: 57 and 77 us at 4,860 on 5,456 states, 91 and 76 at 7,560.
+constexpr int64_t kSmallStates = int64_t(1) << 19;
 struct ExpandArgs {
   uint32_t* table;
   uint64_t mask;
