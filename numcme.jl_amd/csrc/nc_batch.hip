@@ -35,6 +35,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kGran = 256;       // rows of one ownership granule (instances are padded to it)
 constexpr int kCtlBlock = 1024;  // controller workgroup
+constexpr int kCtlInst = kCtlBlock / 16;  // instances whose error sums it folds itself, at most
 constexpr unsigned kMaxRowBlocks = 2048;  // fixed grid of the list-driven row kernels
 constexpr int kChunk = 8;        // iterations per captured graph
 constexpr int kBuildWorkers = 4;  // host threads of nc_batch_create_models
@@ -448,8 +449,8 @@ struct Ctl {
   int n;
   const Params* par;
   const double* t_out;
-  double* err;              // folded error sums of the iteration just run
-  const double* partials;   // not null: the controller folds them itself
+  const double* err;        // folded error sums of the iteration just run
+  const double* partials;   // not null: the controller folds them itself (n <= kCtlInst)
   const int32_t* seg_start;
   int64_t grans;
   const int64_t* nrows;     // error norm length per instance
@@ -562,30 +563,25 @@ __device__ uint32_t block_scan(uint32_t v, uint32_t* sh, uint32_t& total) {
 // with work in the next iteration (a step to take, or an accept / snapshot to apply).
 __global__ __launch_bounds__(kCtlBlock) void k_bcontrol(Ctl c, int init) {
   __shared__ uint32_t sh[kCtlBlock / 64 + 1];
-  __shared__ double s_err[kCtlBlock];
+  __shared__ double s_err[kCtlInst];
   __shared__ int any, changed;
   if (threadIdx.x == 0) any = 0, changed = init;
   __syncthreads();
   const int n_out = c.par->n_out;
   const double h0 = c.par->h0;
   const int64_t max_steps = c.par->max_steps;
-  // the error sums: sixteen lanes an instance, so that up to 64 instances' dependent loads
-  // (range, then partials) are in flight at once
+  // the error sums of up to kCtlInst instances: sixteen lanes each, so that all their
+  // dependent loads (range, then partials) are in flight at once
   if (!init && c.partials) {
-    const int lane = threadIdx.x & 15;
-    for (int i = threadIdx.x >> 4; i < c.n; i += kCtlBlock / 16) {
+    const int lane = threadIdx.x & 15, i = threadIdx.x >> 4;
+    if (i < c.n) {
       double sum = 0.0;
       const int64_t g0 = c.gran_start[i], g1 = c.gran_start[i + 1];
       const int q0 = c.seg_start ? c.seg_start[i] : 0, q1 = c.seg_start ? c.seg_start[i + 1] : 0;
       for (int64_t g = g0 + lane; g < g1; g += 16) sum += c.partials[g];
       for (int q = q0 + lane; q < q1; q += 16) sum += c.partials[c.grans + q];
       for (int off = 8; off > 0; off >>= 1) sum += __shfl_down(sum, off, 16);
-      if (lane == 0) {
-        if (i < kCtlBlock)
-          s_err[i] = sum;
-        else
-          c.err[i] = sum;
-      }
+      if (lane == 0) s_err[i] = sum;
     }
   }
   __syncthreads();
@@ -593,7 +589,7 @@ __global__ __launch_bounds__(kCtlBlock) void k_bcontrol(Ctl c, int init) {
   for (int i = threadIdx.x; i < c.n; i += kCtlBlock) {
     if (!init && c.htry[i] != 0.0) atomicOr(&any, 1);
     control_one(c, i, init != 0, n_out, h0, max_steps,
-                init ? 0.0 : (c.partials && i < kCtlBlock ? s_err[i] : c.err[i]));
+                init ? 0.0 : (c.partials ? s_err[i] : c.err[i]));
     running += c.htry[i] != 0.0;
   }
   // instance offsets into the list, in instance order
@@ -907,10 +903,13 @@ Dev dev_view(nc_batch_s* B) {
 // granule there); the other shapes run the stage and error passes.
 bool fused(const nc_batch_s* B) { return B->rows_per_thread == 4; }
 
-// Up to here the one-workgroup controller folds the error sums itself; more granules are
-// folded by a launch of their own first.
+// Where the one-workgroup controller folds the error sums itself; otherwise a launch of its
+// own folds them first. One round of its sums takes the place of that launch (solves of 16
+// and 64 telegraph instances: 4.1 against 4.3 ms, 4.8 against 5.0; 64 instances in 4,032
+// granules 10.0 against 10.1, in 16,064 34.1 against 33.9). More rounds, one after the other,
+// cost more than it: 600 instances 12.0 against 10.9 ms.
 constexpr int64_t kControllerGrans = 4096;
-bool controller_folds(const nc_batch_s* B) { return B->grans <= kControllerGrans; }
+bool controller_folds(const nc_batch_s* B) { return B->n <= kCtlInst && B->grans <= kControllerGrans; }
 
 Ctl ctl_view(nc_batch_s* B) {
   Ctl c{};

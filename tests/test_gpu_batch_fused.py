@@ -4,7 +4,8 @@ passes (one and two rows per thread).
 The forms share the stage arithmetic; the error norm is summed in another order, so a step
 may differ in its last bits: the solutions agree to the integrator's tolerance. Instances
 lie at the edges of a 256-row granule, single and many, with slot counts 3, 4, 6 and 12,
-computed and loaded columns and empty sink rows.
+computed and loaded columns and empty sink rows. The controller folds the error sums of up to
+64 instances itself; 65 take the separate fold.
 """
 import numpy as np
 import pytest
@@ -26,6 +27,9 @@ def _instances(kind, precision):
     if kind == "edges":
         for n in (1, 2, 125, 126, 127, 128, 129, 254, 256):
             add(S, props, th, np.asarray(models.telegraph_states(n - 1)))
+    elif kind in ("n64", "n65"):
+        for i in range(int(kind[1:])):
+            add(S, props, np.asarray(th) * (1.0 + 0.01 * i), np.asarray(models.telegraph_states(3 + 5 * i)))
     elif kind == "one":
         add(S, props, th, np.asarray(models.telegraph_states(200)))
     else:
@@ -45,7 +49,7 @@ def _instances(kind, precision):
 
 
 @pytest.mark.parametrize("precision,bar", [("fp64", 1e-9), ("fp32", 1e-6)])
-@pytest.mark.parametrize("kind", ["one", "edges", "mixed", "twelve"])
+@pytest.mark.parametrize("kind", ["one", "edges", "mixed", "twelve", "n64", "n65"])
 def test_fused_against_separate(gpu, precision, bar, kind):
     inst = _instances(kind, precision)
     u0s = []
