@@ -551,13 +551,14 @@ void launch_sens(nc_sensmatrix_s* SA, double t, const void* v, int64_t vstride, 
 
 }  // namespace
 
-// With FP64 stage-input copies the epilogue kernel measured 3% slower over a solve of 13
-// blocks on 262,144 states than the separate stage passes (8% faster in FP32 storage); below
-// 2^18 rows in all blocks the passes are launch latency: 13 blocks on 9,216 states took 25.7 ms
-// with them and 20.1 with the epilogue
+// With FP64 stage-input copies the epilogue saves the passes' launches and a re-read, and its
+// larger working set costs occupancy: solves of 13 blocks with it and with the separate passes
+// took 4.7 and 6.0 ms at 120,000 unknowns, 5.2 and 6.0 at 333,000, 7.6 and 8.5 at 852,000, 13.6
+// and 14.8 at 2.08 million, 28.2 and 24.5 to 27.0 at 3.41 million. (FP32 storage: 8% faster
+// with it at the last.) The same bits either way.
 bool sens_rk_fusable(const nc_sensmatrix_s* SA) {
   return SA->P + 1 <= 16 &&
-         (SA->A->precision == NC_FP32 || (int64_t)(SA->P + 1) * SA->A->n_rows <= (int64_t(1) << 18));
+         (SA->A->precision == NC_FP32 || (int64_t)(SA->P + 1) * SA->A->n_rows <= (int64_t(1) << 21));
 }
 
 void sens_matvec_launch(nc_sensmatrix_s* SA, double t, const void* v, int64_t vstride, double* out, int64_t ostride,
