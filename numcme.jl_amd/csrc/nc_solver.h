@@ -92,13 +92,12 @@ inline double krylov_step_tol(const nc_solver_s* S) {
 }
 // Happy breakdown: the residual of the exhausted space is |beta| h per unit time, so h has to
 // fall below the tolerance the caller asks for, per unit time too (Expokit's fixed 1e-7 let
-// solves near a stationary state jump to the next output with 2e-5 of error). In FP64 storage
-// a tenth of it: that jump is most of the error there (300 counts at 1e-6: 1.7e-5 became
-// 1.7e-6 with 28% more steps, the step tolerance above included). In FP32 h does not fall much
-// below 1e-7, and a smaller threshold costs four times the steps.
+// solves near a stationary state jump to the next output with 2e-5 of error), and in FP64
+// storage below 1e-8 at any tolerance: that jump is most of the error there. In FP32 h does
+// not fall much below 1e-7, and a smaller threshold costs four times the steps.
 inline double krylov_breakdown_tol(const nc_solver_s* S) {
-  const double tol = std::min(S->opts.krylov_tol, 1e-7) * (S->vs == 8 ? 0.1 : 1.0);
-  return std::max(tol, 1e-14);
+  const double most = S->vs == 8 ? 1e-8 : 1e-7;
+  return std::max(std::min(S->opts.krylov_tol, most), 1e-14);
 }
 // Error that a step need not go below, relative to |V_0|: the first vector rounded to FP32 is
 // off by about 2^-25 of its norm to begin with. Steps that followed the estimate further down
