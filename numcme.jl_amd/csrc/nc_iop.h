@@ -4,12 +4,20 @@
 // equation H. D. Vo and R. B. Sidje, "Approximating the large sparse matrix exponential
 // using incomplete orthogonalization and Krylov subspaces of variable dimension", Numer.
 // Linear Algebra Appl. 24, 2017): V_{c+1} = A v_c made orthogonal to V_c and V_{c-1} only.
-// A V = V H holds whatever the angles between older vectors, so exp(tau A) u is
-// approximated by V exp(tau H) e1 as with full orthogonalisation, with the same error
-// estimate and step control. A column then reads two basis vectors instead of all of
-// them: the full form's two sweeps over 1..30 vectors took 60% of a solve on the 1024^2
-// toggle switch. Measured step counts are 0-20% above the full form's at equal tolerance
-// (toggle, telegraph, cascade; FP64 and FP32 storage).
+// A V = V H holds, to the rounding of the stored vectors, whatever the angles between older
+// ones, so exp(tau A) u is approximated by V exp(tau H) e1 as with full orthogonalisation, with
+// the same error estimate, held lower (krylov_step_tol). A column then reads two basis vectors
+// instead of all of them: the full form's two sweeps over 1..30 vectors took 60% of a solve on
+// the 1024^2 toggle switch. The price is steps. Full form, this form with the estimate held to
+// the tolerance, and as it is held:
+//   telegraph 800 states   FP64 1e-9    73  102  118     39 ms,   8.8,  10.0
+//   toggle    301 x 259    FP64 1e-12   60   82   94     32 ms,  19.2,  21.5
+//   toggle    1024^2       FP32 1e-9    99  137  123    119 ms,  87.8,  78.5
+//   toggle    1024^2       FP64 1e-9    88  154  194    158 ms, 119.6, 149.9
+// (the breakdown threshold is no part of it: with Expokit's 1e-7 the second column reads 99,
+// 82, 137, 154). Near the stationary state of a stiff box the full form's threshold saved it
+// most steps, at 2e-5 of error: 8,000 telegraph states at 1e-9 FP64 219 and 868 steps, 119 and
+// 163 ms, FP32 164 and 958, 87 and 185 ms.
 //
 // The basis is stored unnormalised with FP64 scales sc_c = 1 / |V_c|. Column c sums
 //   T0 = V_c.q  T1 = V_{c-1}.q  T2 = V_c.V_c  T3 = V_{c-1}.V_c  T4 = q.q,   q = A V_c,

@@ -7,7 +7,8 @@ generator), or, on a small space, with all the others in one workgroup. The form
 arithmetic and the order of the sums: a solve must give the same snapshots bit for bit.
 Sizes lie at the edges of the one-workgroup form's row counts, of the 512-row blocks and of
 the workgroup groups; the generators have 4, 6 and 12 slots, computed, loaded and mixed
-columns, and sink rows of 1 to 700 entries.
+columns, and sink rows of 1 to 700 entries. The errors of FP64 and FP32 solves are held
+against the exact exponential.
 """
 import numpy as np
 import pytest
@@ -208,7 +209,8 @@ def test_near_stationary_states(gpu, n, theta, tol):
     out = _integrate(A, nh.KrylovExpv(m=30, tol=tol, precision="fp64").opts(1e-6, 1e-4), ref, 0.0, ts, space)
     for k in range(K + 1):
         got = np.concatenate([out.p[k].values, out.sinks[k]])
-        # a step accepts 1.2 tol per unit time; the semigroup does not amplify it in the
-        # 1-norm, which 2-norm errors bound within sqrt(N)
-        assert np.linalg.norm(got - ref) <= 1.2 * tol * ts[k] * np.sqrt(N) + 1e-12
+        # per unit time a step accepts 1.2e-3 tol and an exhausted space leaves at most tol, or
+        # 1e-8; the semigroup does not amplify it in the 1-norm, which 2-norm errors bound
+        # within sqrt(N)
+        assert np.linalg.norm(got - ref) <= (1.2e-3 * tol + min(tol, 1e-8)) * ts[k] * np.sqrt(N) + 1e-12
         ref = P @ ref
